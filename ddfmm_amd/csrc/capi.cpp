@@ -124,7 +124,9 @@ static int64_t vbytes(const std::vector<T>& v) { return (int64_t)v.size() * (int
 static void plan_bytes(const HostPlan& h, int precision, int64_t& fixed, int64_t& per_rhs, int64_t& transient) {
     const bool mixed = precision == DDFMM_MIXED || precision == DDFMM_MIXED_SPLIT;
     fixed = vbytes(h.px) + vbytes(h.py) + vbytes(h.pz) + 2 * vbytes(h.perm) + vbytes(h.grid) +
-            h.opmat_total * (int64_t)sizeof(double2) + (mixed ? h.opmat_total * (int64_t)sizeof(float2) : 0) +
+            (h.opmat_total + h.opmat_pad) * (int64_t)sizeof(double2) +
+            (mixed ? (h.prm.pack ? h.opmat_up : h.opmat_total) * (int64_t)sizeof(float2) : 0) +
+            h.pack_total * (int64_t)sizeof(float2) +
             (precision == DDFMM_MIXED_SPLIT ? h.opmat_total * 16 : 0) +
             vbytes(h.ktasks) + vbytes(h.ksrcs) + vbytes(h.groups) + vbytes(h.tiles) + vbytes(h.colB) +
             vbytes(h.colC) + vbytes(h.colA) + vbytes(h.fsrc) + vbytes(h.vtrg) + vbytes(h.vchunk) +
@@ -132,7 +134,8 @@ static void plan_bytes(const HostPlan& h, int precision, int64_t& fixed, int64_t
     const int64_t esz = mixed ? (int64_t)sizeof(float2) : (int64_t)sizeof(double2);
     per_rhs = 2 * h.N * (int64_t)sizeof(double2);
     for (int b = 0; b < BUF_COUNT; ++b) per_rhs += h.bufsize[b] * esz;
-    transient = vbytes(h.genpts) + vbytes(h.kgen);
+    for (int b = 0; b < BUF_COUNT; ++b) fixed += h.bufsize[b] > 0 ? BUF_SLACK * esz : 0;
+    transient = std::max(vbytes(h.genpts) + vbytes(h.kgen), vbytes(h.pack));
 }
 
 // The kernel-apply flavour is fixed per context (each right-hand side then has the same
@@ -264,6 +267,7 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         q.numC = p->numC; q.ktype = p->kernel;
         q.fuse_solves = p->precision != DDFMM_FP64;
         q.nrhs_max = p->nrhs_max;
+        q.pack = p->precision == DDFMM_MIXED;
         // the matrix-core kernel apply (mixed modes, four or more right-hand sides)
         // evaluates near-field leaf pairs of a small leaf once for both directions; with
         // leaves of up to 128 points most pairs qualify (with larger leaves few do, and the
@@ -314,7 +318,10 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
             d.iperm = c->upload(iperm);
         }
         d.grid = c->upload(h.grid);
-        d.opmat = c->alloc<double2>(h.opmat_total);
+        const int64_t table = h.opmat_total + h.opmat_pad;
+        d.opmat = c->alloc<double2>(table);
+        if (h.opmat_pad > 0)
+            HIPCHK(hipMemset(d.opmat + h.opmat_total, 0, (size_t)h.opmat_pad * sizeof(double2)));
         if (!h.opmat.empty())
             HIPCHK(hipMemcpy(d.opmat, h.opmat.data(), h.opmat.size() * sizeof(double2), hipMemcpyHostToDevice));
         d.ktasks = c->upload(h.ktasks); d.ksrcs = c->upload(h.ksrcs);
@@ -346,8 +353,19 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
             HIPCHK(hipStreamSynchronize(c->stream));
         }
         if (d.mixed) {
-            d.opmat32 = c->alloc<float2>(h.opmat_total);
-            HIPCHK(launch_to_f32(d.opmat, d.opmat32, h.opmat_total, c->stream));
+            const int64_t n32 = h.prm.pack ? h.opmat_up : h.opmat_total;
+            d.opmat32 = c->alloc<float2>(n32);
+            HIPCHK(launch_to_f32(d.opmat, d.opmat32, n32, c->stream));
+            if (!h.pack.empty()) {
+                d.oppack = c->alloc<float2>(h.pack_total);
+                PackA* jobs = nullptr;
+                HIPCHK(hipMalloc(&jobs, h.pack.size() * sizeof(PackA)));
+                HIPCHK(hipMemcpy(jobs, h.pack.data(), h.pack.size() * sizeof(PackA), hipMemcpyHostToDevice));
+                // three products (e^{ikr}/r) take k in pairs, four keep the stored order
+                HIPCHK(launch_pack(jobs, (int)h.pack.size(), d.opmat, d.oppack, d.ktype == 0, c->stream));
+                HIPCHK(hipStreamSynchronize(c->stream));
+                HIPCHK(hipFree(jobs));
+            }
             if (c->precision == DDFMM_MIXED_SPLIT) {    // translations as split-BF16 products
                 d.opmatbf = (void*)c->alloc<double2>(h.opmat_total);
                 HIPCHK(launch_to_bf16s(d.opmat, d.opmatbf, h.opmat_total, c->stream));
@@ -357,8 +375,8 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         // work buffers, after the setup-time tables are gone
         for (int b = 0; b < BUF_COUNT; ++b) {
             d.bt.stride[b] = h.bufsize[b];
-            d.bt.p[b] = esz == 8 ? (void*)c->alloc<float2>(h.bufsize[b] * c->slab)
-                                 : (void*)c->alloc<double2>(h.bufsize[b] * c->slab);
+            const int64_t n = h.bufsize[b] > 0 ? h.bufsize[b] * c->slab + BUF_SLACK : 0;
+            d.bt.p[b] = esz == 8 ? (void*)c->alloc<float2>(n) : (void*)c->alloc<double2>(n);
         }
         d.den_io = c->alloc<double2>(h.N * c->slab);
         d.val_io = c->alloc<double2>(h.N * c->slab);
@@ -366,6 +384,7 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         std::vector<cpx>().swap(h.opmat);
         std::vector<double>().swap(h.genpts);
         std::vector<KGen>().swap(h.kgen);
+        std::vector<PackA>().swap(h.pack);
         c->ready = true;
     } catch (const HipFail& e) {
         c->release();

@@ -108,6 +108,21 @@ __device__ __forceinline__ int xcd_item(int b, int n) {
     return x * q + min(x, r) + k;
 }
 
+// The same in chunks of C consecutive items, dealt to the XCDs in turn: neighbours still share
+// an L2, and items whose cost drifts along the list (GEMM groups in order of rank) spread
+// over the XCDs, where eighths of the list left the XCDs with up to a fifth more or less work
+// than the mean (W = 1 L2L of 4M points x 8 RHS: 8.1 -> 7.0 ms by this mapping alone).
+template <int C>
+__device__ __forceinline__ int xcd_chunk(int b, int n) {
+    const int full = n / (8 * C) * (8 * C);
+    if (b >= full) return full + xcd_item(b - full, n - full);
+    const int x = b & 7, k = b >> 3;
+    return (k / C) * 8 * C + x * C + k % C;
+}
+// 64-column tiles per chunk; 64 to 512 measured within 1% of each other, 8 and 32 up to 25%
+// slower at 64 RHS, where one planned tile alone becomes 64 tiles of the same operator
+constexpr int GEMM_XCD_CHUNK = 128;
+
 // ---------------------------------------------------------------- kernel apply
 constexpr int KA_THREADS = 256;
 
@@ -606,176 +621,113 @@ template <> struct Mfma<double> {
 
 constexpr int MAXKB = 8;           // at most 8 K blocks (children of a box)
 
-// LDS layouts: complex values interleaved (one 64-bit (f32) or 128-bit (f64) access per
-// element); every 16-lane (f32) or 8-lane (f64) group of a fragment read touches one
-// contiguous 128-byte row segment or distinct banks:
-//   A slab [k][m], row stride SA = 16 MB + 4 (f32) or + 2 (f64) complex: the 4 k rows
-//   written by 4 neighbouring lanes in the transposed-A store land in distinct banks;
-//   B slab [n][k], row stride SB = 17 (odd: 16 columns at one k in distinct banks).
-template <class R> struct Lds;
-template <> struct Lds<float> { static constexpr int SAPAD = 4; using C = float2; };
-template <> struct Lds<double> { static constexpr int SAPAD = 2; using C = double2; };
-
 // C[:, ccol] (=|+=) diag(scale) * op(A) * B[:, bcol] on MFMA 16x16x4 (f32 or f64).
-// A tile covers MB row blocks of 16 (the group's rows split evenly over its tiles; tiles
-// are launched per MB) and GEMM_TN = 64 columns, 16 per wave; complex products as four
-// real MFMAs.  K runs over segments (the whole K, or the K blocks present in at least
-// one of the tile's columns) in slabs of 16 with a register-prefetch pipeline: slab s+1
-// is loaded while slab s runs on the matrix cores.  Padding stays within 16 rows, 4 k
-// and 16 columns: the MFMAs stop at the last k step of a segment, and a wave whose
-// columns are all empty, or all lack the current K block, skips the segment's MFMAs.
-template <class TA, class V, class R, int MB, bool G3M = false>
-__global__ __launch_bounds__(256) void gemm_kernel(
+// A block covers MB row blocks of 16 (the group's rows split evenly over its tiles; tiles
+// are launched per MB) and 64 CB columns; each of its four waves owns 16 CB columns and
+// works alone: operands go straight from memory (A from L2 and L1, where the block's waves
+// meet) into the MFMA registers, one pipeline step of KQ k steps ahead, with no LDS staging
+// and no barriers.  K runs over segments: the whole K, or the K blocks present in at least
+// one of the wave's columns.
+//
+// What bounds it: the vector memory path.  With its loads taken out the loop runs at 143 of
+// the 155 TF/s that the f32 matrix cores sustain here; A in the stored order (ten 8-byte
+// loads per 30 MFMAs, each over four half-filled line groups) held it at 98, packed A (five
+// 16-byte loads of a contiguous KiB) brings it to 120.  Staging through LDS (two buffers,
+// one barrier per 16 k) reached 85 to 101: 124 with neither loads nor stores, as its waves
+// stall together at the barriers.  Translations alone, LDS form -> this one: 4M points x 8
+// RHS 28.9 -> 23.4 ms, 250k x 64 RHS 58.9 -> 43.7 ms, 1M x 1 RHS 5.9 -> 4.5 ms.
+//
+// Bounds of the loads: A is read without predicates; rows past the group's last one and k
+// past a segment's end read on into the table, whose end is padded with zeros (opmat_pad), or
+// a packed block's zeros; such rows are not stored, and such k meet zeros in B.  B is clamped
+// to the segment, and entries past it and those of absent columns (which read the buffer's
+// start) are replaced by zeros.  A column's order of k depends on G3M alone, so neither MB
+// nor CB changes a bit (the instruction itself sums its k in order by fma).
+// Two adjacent FP32 complex values by one 16-byte load (global loads need dword alignment
+// only).
+struct CPair {
+    float2 e[2];
+};
+__device__ __forceinline__ CPair load_pair(const float2* p) {
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
+    const f4u r = *(const f4u*)p;
+    return {{make_float2(r.x, r.y), make_float2(r.z, r.w)}};
+}
+
+// A's form: as stored (column-major blocks), transposed as stored, or packed (FP32, PackA in
+// plan.hpp) in the order the lanes take it.
+enum GemmA : int { GEMM_A = 0, GEMM_AT = 1, GEMM_APACK = 2 };
+
+template <class TA, class V, class R, int MB, int CB, int AF, bool G3M>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(
     const GGroup* __restrict__ groups, const GTile* __restrict__ tiles,
     const int64_t* __restrict__ colB, const int64_t* __restrict__ colC, const int64_t* __restrict__ colA,
     const TA* __restrict__ opm, BufTable bt, int tile0, int nr) {
     using M = Mfma<R>;
     using T = typename Real<V>::T;
-    using RC = typename Lds<R>::C;
-    constexpr int KS = 16, TM = 16 * MB, SA = TM + Lds<R>::SAPAD, SB = 17;
-    constexpr int NA = TM * KS / 256, NB = GEMM_TN * KS / 256;   // elements per thread and slab
+    constexpr int TN = GEMM_TN * CB;
+    constexpr bool TRANS = AF == GEMM_AT, PACK = AF == GEMM_APACK;
+    constexpr int KQ = PACK ? 2 : 1, KS = 4 * KQ;      // k steps and k per pipeline step
+    // k order of a pipeline step: with three products lane group lk takes k = 2 lk + q in k
+    // step q (one 16-byte load of B; a last step of at most 4 k runs k = lk alone), with four
+    // k = lk + 4 q
+    constexpr bool PAIR = PACK && G3M;
     // columns are (box, rhs) pairs, rhs fastest: column n is box n / nr of the group in
     // right-hand side n % nr (that rhs slab of the buffer).  A planned tile (GEMM_TN boxes)
-    // becomes nr launched tiles of GEMM_TN such columns; those past the group's last
-    // column exit at once.
-    const int bx = xcd_item(blockIdx.x, gridDim.x);
-    GTile tl = tiles[tile0 + bx / nr];
+    // becomes ceil(nr / CB) launched tiles of TN such columns; waves past its boxes or the
+    // group's last column exit at once.
+    const int per = (nr + CB - 1) / CB;
+    const int bx = xcd_chunk<GEMM_XCD_CHUNK / CB>(blockIdx.x, gridDim.x);
+    const GTile tl = tiles[tile0 + bx / per];
     const GGroup g = groups[tl.g];
-    const int ncx = g.ncols * nr;
-    tl.n0 = tl.n0 * nr + GEMM_TN * (bx % nr);
-    if (tl.n0 >= ncx) return;
+    const int ncx = min(g.ncols, tl.n0 + GEMM_TN) * nr;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int n0 = tl.n0 * nr + TN * (bx % per) + 16 * CB * wave;    // the wave's first column
+    if (n0 >= ncx) return;
     const V* B = bufp<V>(bt, g.bbuf);
     V* C = bufp<V>(bt, g.cbuf);
     const int64_t sB = bt.stride[g.bbuf], sC = bt.stride[g.cbuf];
-    // f32: two LDS slab buffers (one barrier per slab); f64 slabs are twice the size and
-    // take twice the MFMA time per k, so one buffer and two barriers per slab
-    constexpr int NBUF = sizeof(R) == 4 ? 2 : 1;
-    __shared__ RC As[NBUF][KS * SA];
-    __shared__ RC Bs[NBUF][GEMM_TN * SB];
-    __shared__ int64_t bo[MAXKB][GEMM_TN];   // B offset of (block, column), -1 = absent
-    __shared__ int64_t ao[MAXKB];            // A offset of each active segment
-    __shared__ int used[MAXKB][4], act[MAXKB], wm[MAXKB], nact_s;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int li = lane & 15, lk = lane >> 4;
     const int kb = g.kb ? g.kb : g.K;                   // segment length
     const int nkb = g.kb ? g.K / g.kb : 1;
+    // B offsets of the wave's columns per K block, -1 = absent: written and read by this wave
+    __shared__ int64_t bo[4][MAXKB][16 * CB];
 
-    // per-thread slab elements, fixed for the tile: A (row, k) and B (k, column)
-    const int mrows = g.M - tl.m0;                      // rows >= mrows are zero
-    const int64_t kstride = g.transA ? 1 : g.lda;       // A offset per k
-    int64_t aoffs[NA];
-    int akk[NA], alds[NA];
+    int64_t coff[CB];                                   // this lane's output columns
+    unsigned act = 0;                                   // segments with a present column
+    {
+        int64_t base[CB], rs[CB];
 #pragma unroll
-    for (int l = 0; l < NA; ++l) {
-        const int e = tid + 256 * l;
-        int mm, kk;
-        if (g.transA) {              // global A[k + m*lda]: 4 consecutive k per row
-            kk = (e & 3) | ((e / (4 * TM)) << 2);
-            mm = (e >> 2) % TM;
-        } else {                     // global A[m + k*lda]: consecutive rows
-            mm = e % TM;
-            kk = e / TM;
+        for (int c = 0; c < CB; ++c) {
+            const int n = n0 + 16 * c + li;
+            const int box = n / nr, r = n - box * nr;
+            base[c] = n < ncx ? g.bcol0 + (int64_t)box * nkb : -1;
+            rs[c] = r * sB;
+            coff[c] = n < ncx ? colC[g.col0 + box] + r * sC : -1;
         }
-        const int64_t m = tl.m0 + mm;
-        aoffs[l] = g.transA ? kk + m * g.lda : m + kk * (int64_t)g.lda;
-        akk[l] = mm < mrows ? kk : KS;                  // KS: never loaded
-        alds[l] = kk * SA + mm;
-    }
-    int64_t bc[NB];                                     // column offsets of the current segment
-    int bkk[NB], blds[NB];
 #pragma unroll
-    for (int l = 0; l < NB; ++l) {
-        const int e = tid + 256 * l;
-        bkk[l] = e % KS;
-        blds[l] = (e / KS) * SB + (e % KS);
-    }
-    // this lane's output column, fetched early (the epilogue needs it last)
-    const int ncol = tl.n0 + wave * 16 + li;
-    const int64_t coff = ncol < ncx ? colC[g.col0 + ncol / nr] + (int64_t)(ncol % nr) * sC : -1;
-
-    // segments.  Contiguous B (kb = 0): one segment, column offsets read straight into
-    // registers, waves with columns run.  Blocked B: a table of the K blocks present in
-    // the tile's columns, with per-wave masks.
-    int nact = 1, wm0 = 0;
-    if (g.kb == 0) {
-        const int nv = ncx - tl.n0;
-        wm0 = nv >= GEMM_TN ? 15 : (1 << ((nv + 15) >> 4)) - 1;
+        for (int t = 0; t < MAXKB / 4; ++t) {
+            const int h = 4 * t + lk;
+            bool any = false;
 #pragma unroll
-        for (int l = 0; l < NB; ++l) {
-            const int n = tl.n0 + (tid + 256 * l) / KS;
-            bc[l] = n < ncx ? colB[g.bcol0 + n / nr] + (int64_t)(n % nr) * sB : -1;
-        }
-    } else {
-        if (tid < MAXKB * 4) used[tid >> 2][tid & 3] = 0;
-        __syncthreads();
-        for (int e = tid; e < nkb * GEMM_TN; e += 256) {
-            const int h = e / GEMM_TN, j = e % GEMM_TN;
-            const int n = tl.n0 + j;
-            int64_t v = n < ncx ? colB[g.bcol0 + (int64_t)(n / nr) * nkb + h] : -1;
-            if (v >= 0) v += (int64_t)(n % nr) * sB;
-            bo[h][j] = v;
-            if (v >= 0) used[h][j >> 4] = 1;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            int c = 0;
-            for (int h = 0; h < nkb; ++h) {
-                const int w = used[h][0] | (used[h][1] << 1) | (used[h][2] << 2) | (used[h][3] << 3);
-                if (w) {
-                    act[c] = h;
-                    wm[c] = w;
-                    ++c;
-                }
+            for (int c = 0; c < CB; ++c) {
+                int64_t v = base[c] >= 0 && h < nkb ? colB[base[c] + h] : -1;
+                any |= v >= 0;
+                bo[wave][h][16 * c + li] = v >= 0 ? v + rs[c] : -1;
             }
-            nact_s = c;
+            const uint64_t m = __ballot(any);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if ((m >> (16 * q)) & 0xffff) act |= 1u << (4 * t + q);
         }
-        __syncthreads();
-        nact = nact_s;
-        if (tid < nact) ao[tid] = colA[g.acol0 + act[tid]];
-        __syncthreads();
+        wave_lds_order();
     }
-    TA ra[NA];
-    V rb[NB];
-    auto load = [&](int i, int k0, bool newseg) {
-        const TA* Ab = opm + (g.kb ? ao[i] : g.aoff) + k0 * kstride;
-        const int kl = kb - k0;
-        if (newseg) {
+    const unsigned lda = g.lda;
+    unsigned ao[TRANS ? MB : 1];                        // this lane's A offset (of each row block)
 #pragma unroll
-            for (int l = 0; l < NB; ++l) bc[l] = bo[act[i]][(tid + 256 * l) / KS];
-        }
-#pragma unroll
-        for (int l = 0; l < NA; ++l) {
-            TA a;
-            a.x = 0;
-            a.y = 0;
-            if (akk[l] < kl) a = Ab[aoffs[l]];
-            ra[l] = a;
-        }
-        const V* Bk = B + k0;
-#pragma unroll
-        for (int l = 0; l < NB; ++l) {
-            V b = mk<V>(0, 0);
-            if (bc[l] >= 0 && bkk[l] < kl) b = Bk[bc[l] + bkk[l]];
-            rb[l] = b;
-        }
-    };
-    auto store = [&](int q) {
-#pragma unroll
-        for (int l = 0; l < NA; ++l) {
-            RC v;
-            v.x = (R)ra[l].x;
-            v.y = (R)ra[l].y;
-            As[q][alds[l]] = v;
-        }
-#pragma unroll
-        for (int l = 0; l < NB; ++l) {
-            RC v;
-            v.x = (R)rb[l].x;
-            v.y = (R)rb[l].y;
-            Bs[q][blds[l]] = v;
-        }
-    };
+    for (int a = 0; a < (TRANS ? MB : 1); ++a)
+        ao[a] = PACK ? 2 * lane : TRANS ? (16 * a + li) * lda + lk : lk * lda + li;
+    const unsigned kstep = PACK ? 128 * lda : TRANS ? KS : KS * lda;    // A elements per pipeline step
 
     // G3M (FP32 contexts of the e^{ikr}/r kernel): three real products per complex one,
     // summed over k apart: k1 = (Ar + Ai) Br, k2 = Ar (Bi - Br), k3 = Ai (Br + Bi); Re C =
@@ -784,155 +736,255 @@ __global__ __launch_bounds__(256) void gemm_kernel(
     // equivalent densities then lose accuracy, so it keeps four products (Re C in cr, Im C
     // in ci), as FP64 does.
     static_assert(!G3M || sizeof(R) == 4, "three products in FP32 only");
-    typename M::acc4 cr[MB], ci[MB], c3[G3M ? MB : 1];
+    typename M::acc4 cr[CB][MB], ci[CB][MB], c3[CB][G3M ? MB : 1];
 #pragma unroll
-    for (int a = 0; a < MB; ++a)
+    for (int c = 0; c < CB; ++c)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            cr[a][v] = 0;
-            ci[a][v] = 0;
-            if constexpr (G3M) c3[a][v] = 0;
-        }
+        for (int a = 0; a < MB; ++a)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                cr[c][a][v] = 0;
+                ci[c][a][v] = 0;
+                if constexpr (G3M) c3[c][a][v] = 0;
+            }
 
-    const int bb = (wave * 16 + li) * SB + lk, aa = lk * SA + li;
-    // MFMAs of slab (i, k0) from LDS buffer q: four sweeps over the row blocks per k step,
-    // so consecutive MFMAs never accumulate into the same registers
-    auto mfma_slab = [&](int i, int k0, int q) {
-        if (!((((g.kb ? wm[i] : wm0)) >> wave) & 1)) return;
-        const int nsteps = (min(KS, kb - k0) + 3) >> 2;
-        for (int s = 0; s < nsteps; ++s) {
-            const RC bv = Bs[q][bb + 4 * s];
-            const R br = bv.x, bi = bv.y, mbi = -bi;
-            R ar[MB], ai[MB];
+    struct Step {                  // operands of one pipeline step
+        TA a[KQ][MB];
+        V b[KQ][CB];
+        bool p[CB];                // the column is present in the segment
+        int kl;                    // k left in the segment
+        bool fix;                  // some entry of b must be zeroed
+    };
+    // loader: the current segment's A position and columns, and the k range of the step
+    const TA* Ap = nullptr;
+    const V* Bp[CB];
+    bool pres[CB];
+    bool allp = true;
+    int k0 = 0, kl = 0;            // first k of the step and k left in the segment
+    auto segment = [&]() {
+        const int h = __builtin_ctz(act);
+        act &= act - 1;
+        Ap = opm + (g.kb ? colA[g.acol0 + h] : g.aoff) + (TRANS ? (int64_t)tl.m0 * lda : PACK ? 8 * tl.m0 : tl.m0);
+        k0 = 0;
+        kl = kb;
+        bool all = true;
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+            const int64_t v = bo[wave][h][16 * c + li];
+            pres[c] = v >= 0;
+            all &= v >= 0;
+            Bp[c] = B + (v >= 0 ? v : 0);
+        }
+        allp = __all(all);
+    };
+    auto advance = [&]() {         // false: there is no further step (the loader stays)
+        if (kl > KS) {
+            k0 += KS;
+            kl -= KS;
+            Ap += kstep;
+            return true;
+        }
+        if (!act) return false;
+        segment();
+        return true;
+    };
+    // The loads of a step are unconditional and in one block (past the last step they repeat
+    // it), so that the waits before their use count the next step's loads as outstanding.
+    auto fetch = [&](Step& s) {
+        if constexpr (PAIR) {
+            // the pair's second entry is at most kb (BUF_SLACK)
+            const int k = min(k0 + (kl <= 4 ? lk : 2 * lk), kb - 1);
+#pragma unroll
+            for (int c = 0; c < CB; ++c) {
+                const CPair b = load_pair(Bp[c] + k);
+                s.b[0][c] = b.e[0];
+                s.b[KQ - 1][c] = b.e[1];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < KQ; ++q) {
+                const int k = min(k0 + 4 * q + lk, kb - 1);
+#pragma unroll
+                for (int c = 0; c < CB; ++c) s.b[q][c] = Bp[c][k];
+            }
+        }
+        if constexpr (PACK) {
 #pragma unroll
             for (int a = 0; a < MB; ++a) {
-                const RC av = As[q][aa + 4 * s * SA + 16 * a];
-                ar[a] = av.x;
-                ai[a] = av.y;
+                const float4 v = *(const float4*)(Ap + 128 * a + ao[0]);
+                s.a[0][a] = make_float2(v.x, v.y);
+                s.a[KQ - 1][a] = make_float2(v.z, v.w);
             }
-            if constexpr (G3M) {   // cr = sum k1, ci = sum k2, c3 = sum k3
-                const R bd = bi - br, bs = br + bi;
+        } else {
+            const TA* ap = Ap + ao[0];
 #pragma unroll
-                for (int a = 0; a < MB; ++a) cr[a] = M::op(ar[a] + ai[a], br, cr[a]);
+            for (int a = 0; a < MB; ++a) s.a[0][a] = TRANS ? Ap[ao[TRANS ? a : 0]] : ap[16 * a];
+        }
 #pragma unroll
-                for (int a = 0; a < MB; ++a) ci[a] = M::op(ar[a], bd, ci[a]);
+        for (int c = 0; c < CB; ++c) s.p[c] = pres[c];
+        s.kl = kl;
+        s.fix = kl < KS || !allp;
+    };
+    // sweeps over the row blocks, so consecutive MFMAs never accumulate into the same
+    // registers; one row fragment serves the wave's CB column blocks
+    auto compute = [&](Step& s) {
+        if (s.fix) {
 #pragma unroll
-                for (int a = 0; a < MB; ++a) c3[a] = M::op(ai[a], bs, c3[a]);
-            } else {
+            for (int q = 0; q < KQ; ++q)
 #pragma unroll
-                for (int a = 0; a < MB; ++a) cr[a] = M::op(ar[a], br, cr[a]);
+                for (int c = 0; c < CB; ++c)
+                    if (!s.p[c] || (PAIR && s.kl > 4 ? 2 * lk + q : 4 * q + lk) >= s.kl) s.b[q][c] = mk<V>(0, 0);
+        }
 #pragma unroll
-                for (int a = 0; a < MB; ++a) ci[a] = M::op(ar[a], bi, ci[a]);
+        for (int q = 0; q < KQ; ++q) {
+            if (q > 0 && s.kl <= 4 * q) break;
 #pragma unroll
-                for (int a = 0; a < MB; ++a) cr[a] = M::op(ai[a], mbi, cr[a]);
+            for (int c = 0; c < CB; ++c) {
+                const R br = (R)s.b[q][c].x, bi = (R)s.b[q][c].y;
+                if constexpr (G3M) {   // cr = sum k1, ci = sum k2, c3 = sum k3
+                    const R bd = bi - br, bs = br + bi;
 #pragma unroll
-                for (int a = 0; a < MB; ++a) ci[a] = M::op(ai[a], br, ci[a]);
+                    for (int a = 0; a < MB; ++a) ci[c][a] = M::op((R)s.a[q][a].x, bd, ci[c][a]);
+#pragma unroll
+                    for (int a = 0; a < MB; ++a) c3[c][a] = M::op((R)s.a[q][a].y, bs, c3[c][a]);
+#pragma unroll
+                    for (int a = 0; a < MB; ++a) cr[c][a] = M::op((R)s.a[q][a].x + (R)s.a[q][a].y, br, cr[c][a]);
+                } else {
+                    const R mbi = -bi;
+#pragma unroll
+                    for (int a = 0; a < MB; ++a) cr[c][a] = M::op((R)s.a[q][a].x, br, cr[c][a]);
+#pragma unroll
+                    for (int a = 0; a < MB; ++a) ci[c][a] = M::op((R)s.a[q][a].x, bi, ci[c][a]);
+#pragma unroll
+                    for (int a = 0; a < MB; ++a) cr[c][a] = M::op((R)s.a[q][a].y, mbi, cr[c][a]);
+#pragma unroll
+                    for (int a = 0; a < MB; ++a) ci[c][a] = M::op((R)s.a[q][a].y, br, ci[c][a]);
+                }
             }
         }
     };
-    auto next = [&](int i, int k0, int& ni, int& nk0) {
-        ni = i;
-        nk0 = k0 + KS;
-        if (nk0 >= kb) {
-            ni = i + 1;
-            nk0 = 0;
-        }
-    };
-    if (nact > 0) {
-        load(0, 0, g.kb != 0);
-        store(0);
-    }
-    int i = 0, k0 = 0;
-    if constexpr (NBUF == 2) {
-        // slab s+1 waits in registers while slab s runs; it is written to the other buffer
-        // after the MFMAs, then slab s+2 is fetched; one barrier per slab
-        int ni, nk0;
-        next(i, k0, ni, nk0);
-        bool more = ni < nact;
-        if (more) load(ni, nk0, ni != i);
-        __syncthreads();
-        int q = 0;
-        while (i < nact) {
-            mfma_slab(i, k0, q);
-            int n2i = nact, n2k0 = 0;
-            bool more2 = false;
-            if (more) {
-                store(q ^ 1);
-                next(ni, nk0, n2i, n2k0);
-                more2 = n2i < nact;
-                if (more2) load(n2i, n2k0, n2i != ni);
-            }
-            __syncthreads();
-            i = ni;
-            k0 = nk0;
-            ni = n2i;
-            nk0 = n2k0;
-            more = more2;
-            q ^= 1;
-        }
-    } else {
-        __syncthreads();
-        while (i < nact) {
-            int ni, nk0;
-            next(i, k0, ni, nk0);
-            const bool more = ni < nact;
-            if (more) load(ni, nk0, ni != i);   // global loads in flight during the MFMAs below
-            mfma_slab(i, k0, 0);
-            __syncthreads();
-            if (more) {
-                store(0);
-                __syncthreads();
-            }
-            i = ni;
-            k0 = nk0;
+    if (act) {
+        Step s0, s1;
+        segment();
+        fetch(s0);
+        while (true) {             // the next step's loads are in flight during this one's MFMAs
+            const bool second = advance();
+            fetch(s1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(s0);
+            const bool more = second && advance();
+            fetch(s0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (second) compute(s1);
+            if (!more) break;
         }
     }
     // D layout of a 16x16 MFMA tile: lane holds rows M::row(lane/16, v), column lane%16
-    if (coff < 0) return;
-    V* Cc = C + coff;
 #pragma unroll
-    for (int a = 0; a < MB; ++a) {
+    for (int c = 0; c < CB; ++c) {
+        if (coff[c] < 0) continue;
+        V* Cc = C + coff[c];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int m = tl.m0 + 16 * a + M::row(lk, v);
-            if (m >= g.M) continue;
-            R re = cr[a][v], im = ci[a][v];
-            if constexpr (G3M) {
-                re = cr[a][v] - c3[a][v];
-                im = cr[a][v] + ci[a][v];
+        for (int a = 0; a < MB; ++a) {
+            R re[4], im[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                re[v] = cr[c][a][v];
+                im[v] = ci[c][a][v];
+                if constexpr (G3M) {
+                    re[v] = cr[c][a][v] - c3[c][a][v];
+                    im[v] = cr[c][a][v] + ci[c][a][v];
+                }
             }
-            if (g.soff >= 0) {
-                const TA s = opm[g.soff + m];
-                const R sr = (R)s.x, si = (R)s.y;
-                const R t = re * sr - im * si;
-                im = re * si + im * sr;
-                re = t;
+            if constexpr (sizeof(R) == 4) {      // four adjacent rows: two 16-byte stores
+                typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
+                const int m = tl.m0 + 16 * a + 4 * lk;
+                if (g.soff < 0 && g.mode == 0 && m + 3 < g.M) {
+                    f4u lo = {re[0], im[0], re[1], im[1]}, hi = {re[2], im[2], re[3], im[3]};
+                    *(f4u*)(Cc + m) = lo;
+                    *(f4u*)(Cc + m + 2) = hi;
+                    continue;
+                }
             }
-            if (g.mode == 0) {
-                Cc[m] = mk<V>(re, im);
-            } else {
-                V o = Cc[m];
-                o.x += (T)re;
-                o.y += (T)im;
-                Cc[m] = o;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int m = tl.m0 + 16 * a + M::row(lk, v);
+                if (m >= g.M) continue;
+                R x = re[v], y = im[v];
+                if (g.soff >= 0) {
+                    const TA s = opm[g.soff + m];
+                    const R sr = (R)s.x, si = (R)s.y;
+                    const R t = x * sr - y * si;
+                    y = x * si + y * sr;
+                    x = t;
+                }
+                if (g.mode == 0) {
+                    Cc[m] = mk<V>(x, y);
+                } else {
+                    V o = Cc[m];
+                    o.x += (T)x;
+                    o.y += (T)y;
+                    Cc[m] = o;
+                }
             }
         }
     }
 }
 
-template <class TA, class V, class R, bool G3M = false>
-void launch_gemm(int mb, int n, int nrhs, hipStream_t st, const DevPlan& d, const TA* opm, int t0) {
-    const dim3 grid(n * nrhs, 1);
-#define DDFMM_GEMM_MB(X)                                                                                     \
-    case X:                                                                                                  \
-        gemm_kernel<TA, V, R, X, G3M><<<grid, 256, 0, st>>>(d.groups, d.tiles, d.colB, d.colC, d.colA, opm, \
-                                                            d.bt, t0, nrhs);                                 \
+template <class TA, class V, class R, int CB, int AF, bool G3M>
+void launch_gemm_form(int mb, int n, int nrhs, hipStream_t st, const DevPlan& d, const TA* opm, int t0) {
+    const dim3 grid(n * ((nrhs + CB - 1) / CB), 1);
+#define DDFMM_GEMM_MB(X)                                                                                          \
+    case X:                                                                                                       \
+        gemm_kernel<TA, V, R, X, CB, AF, G3M><<<grid, 256, 0, st>>>(d.groups, d.tiles, d.colB, d.colC, d.colA,   \
+                                                                    opm, d.bt, t0, nrhs);                        \
         break;
     switch (mb) {
         DDFMM_GEMM_MB(1) DDFMM_GEMM_MB(2) DDFMM_GEMM_MB(3) DDFMM_GEMM_MB(4) DDFMM_GEMM_MB(5)
         DDFMM_GEMM_MB(6) DDFMM_GEMM_MB(7)
     }
 #undef DDFMM_GEMM_MB
+}
+
+// FP64 products on operators as stored.
+template <class V>
+void launch_gemm64(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
+    const int n = s.end - s.begin;
+    if (s.trans) launch_gemm_form<double2, V, double, 1, GEMM_AT, false>(s.mb, n, nrhs, st, d, d.opmat, s.begin);
+    else launch_gemm_form<double2, V, double, 1, GEMM_A, false>(s.mb, n, nrhs, st, d, d.opmat, s.begin);
+}
+
+// FP32 products on packed operators.  Two column blocks per wave (CB = 2) halve the operator
+// traffic per product but leave two waves per SIMD and take the union of twice the columns'
+// K blocks: they pay where K is not blocked and the columns of a box fill a wave (32 RHS and
+// up; M2L and W > 1 L2L at 64 RHS 13.7 -> 13.2 ms, at 8 and 16 RHS the same or slower, K-blocked
+// U2U 17.3 -> 18.1 ms) and the launch still has four blocks per CU.
+template <bool G3M>
+void launch_gemm32(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
+    const int n = s.end - s.begin;
+    if (nrhs >= 32 && !s.kblocked && (int64_t)n * nrhs / 2 >= 1024 && s.mb < GEMM_MB)
+        launch_gemm_form<float2, float2, float, 2, GEMM_APACK, G3M>(s.mb, n, nrhs, st, d, d.oppack, s.begin);
+    else
+        launch_gemm_form<float2, float2, float, 1, GEMM_APACK, G3M>(s.mb, n, nrhs, st, d, d.oppack, s.begin);
+}
+
+// One packed operator block per job (PackA): rows in blocks of 16 and k in steps of 8, zeros
+// past the block's edges.
+__global__ __launch_bounds__(256) void pack_kernel(const PackA* __restrict__ jobs, const double2* __restrict__ opmat,
+                                                   float2* __restrict__ out, int pair) {
+    const PackA p = jobs[blockIdx.x];
+    const int nrb = (p.M + 15) / 16, nk = (p.K + 7) / 8;
+    for (int e = threadIdx.x; e < nrb * nk * 128; e += 256) {
+        const int q = e & 1, lane = (e >> 1) & 63, rb = (e >> 7) % nrb, o = (e >> 7) / nrb;
+        const int m = 16 * rb + (lane & 15), lk = lane >> 4;
+        const int k = 8 * o + (pair && p.K - 8 * o > 4 ? 2 * lk + q : lk + 4 * q);
+        float2 v = make_float2(0.f, 0.f);
+        if (m < p.M && k < p.K) {
+            const double2 a = opmat[p.src + (p.trans ? k + (int64_t)m * p.lda : m + (int64_t)k * p.lda)];
+            v = make_float2((float)a.x, (float)a.y);
+        }
+        out[p.dst + e] = v;
+    }
 }
 
 // ---------------------------------------------------------------- split-BF16 complex GEMM (MFMA)
@@ -1863,15 +1915,15 @@ hipError_t launch_stage_t(const DevPlan& d, const Stage& s, int nrhs, hipStream_
     case ST_GEMM:
         if (s.mb < 1 || s.mb > GEMM_MB) return hipErrorInvalidValue;
         if (d.mixed && s.prec == PREC_SOLVE)
-            launch_gemm<double2, float2, double>(s.mb, n, nrhs, st, d, d.opmat, s.begin);
+            launch_gemm64<float2>(s, nrhs, st, d);
         else if (d.mixed && d.opmatbf)
             launch_gemm_bf16s(s.mb, n, nrhs, st, d, s.begin);
         else if (d.mixed && d.ktype == 0)    // e^{ikr}/r: three real products per complex one
-            launch_gemm<float2, float2, float, true>(s.mb, n, nrhs, st, d, d.opmat32, s.begin);
+            launch_gemm32<true>(s, nrhs, st, d);
         else if (d.mixed)
-            launch_gemm<float2, float2, float>(s.mb, n, nrhs, st, d, d.opmat32, s.begin);
+            launch_gemm32<false>(s, nrhs, st, d);
         else
-            launch_gemm<double2, double2, double>(s.mb, n, nrhs, st, d, d.opmat, s.begin);
+            launch_gemm64<double2>(s, nrhs, st, d);
         break;
     case ST_FFTFWD:
         if (d.P != 6) return hipErrorInvalidValue;
@@ -1944,7 +1996,7 @@ hipError_t launch_stage(const DevPlan& d, const Stage& s, int nrhs, hipStream_t 
 
 hipError_t launch_setup_gemm(const DevPlan& d, const Stage& s, hipStream_t st) {
     if (s.kind != ST_GEMM || s.mb < 1 || s.mb > GEMM_MB) return hipErrorInvalidValue;
-    launch_gemm<double2, double2, double>(s.mb, s.end - s.begin, 1, st, d, d.opmat, s.begin);
+    launch_gemm64<double2>(s, 1, st, d);
     return hipGetLastError();
 }
 
@@ -1953,6 +2005,12 @@ hipError_t launch_kgen(const KGen* jobs, int njobs, const double* gp, double2* o
         int n = std::min(65536, njobs - j0);
         kgen_kernel<<<n, 256, 0, st>>>(jobs, gp, opmat, j0, ktype);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_pack(const PackA* jobs, int njobs, const double2* opmat, float2* out, int pair, hipStream_t st) {
+    for (int j0 = 0; j0 < njobs; j0 += 65536)
+        pack_kernel<<<std::min(65536, njobs - j0), 256, 0, st>>>(jobs + j0, opmat, out, pair);
     return hipGetLastError();
 }
 

@@ -327,6 +327,8 @@ struct Builder {
             if (pl.tiles[t].mb < 1 || pl.tiles[t].mb > GEMM_MB) throw Error("internal: tile height out of range");
             Stage q = s;
             q.begin = t; q.end = u; q.mb = pl.tiles[t].mb;
+            q.trans = pl.groups[pl.tiles[t].g].transA;
+            q.kblocked = pl.groups[pl.tiles[t].g].kb > 0;
             dst.push_back(q);
             t = u;
         }
@@ -474,6 +476,7 @@ struct Builder {
     void stages_hf_downward();
     void stages_lf_downward();
     void stages_leaf();
+    void pack_operators();
     void finish(bool want_dump);
 
     // Every descriptor's element range must lie inside the buffer or table it indexes: the
@@ -488,7 +491,10 @@ struct Builder {
             need(st.begin >= 0 && st.begin <= st.end, "stage range");
             if (st.kind == ST_GEMM) {
                 need(st.end <= (int64_t)pl.tiles.size(), "gemm stage");
-                for (int t = st.begin; t < st.end; ++t) need(pl.tiles[t].mb == st.mb, "gemm stage tile height");
+                for (int t = st.begin; t < st.end; ++t) {
+                    need(pl.tiles[t].mb == st.mb, "gemm stage tile height");
+                    need(pl.groups[pl.tiles[t].g].transA == st.trans, "gemm stage operand order");
+                }
             }
             if (st.kind == ST_KAPPLY) need(st.end <= (int64_t)pl.ktasks.size(), "kapply stage");
             if (st.kind == ST_FFTFWD) need(st.end <= (int64_t)pl.fsrc.size(), "fft stage");
@@ -547,6 +553,7 @@ struct Builder {
             for (int t = st.begin; t < st.end; ++t) {
                 need(pl.tiles[t].mb == st.mb, "setup tile height");
                 const GGroup& g = pl.groups[pl.tiles[t].g];
+                need(g.transA == st.trans, "setup operand order");
                 need(g.bbuf == BUF_OPMAT && g.cbuf == BUF_OPMAT, "setup buffers");
             }
         }
@@ -559,9 +566,16 @@ struct Builder {
             }
             if (g.soff >= 0) need(g.soff + g.M <= pl.opmat_total, "gemm row scale");
             auto a_ok = [&](int64_t aoff, int kcols) {
+                if (g.transA == 2)
+                    return aoff >= 0 && aoff % 128 == 0 && g.lda == (g.M + 15) / 16 &&
+                           aoff + (int64_t)((kcols + 7) / 8) * g.lda * 128 <= pl.pack_total;
                 const int64_t last = g.transA ? aoff + (int64_t)(g.M - 1) * g.lda + kcols
                                               : aoff + (int64_t)(kcols - 1) * g.lda + g.M;
-                return aoff >= 0 && last <= pl.opmat_total && g.lda >= (g.transA ? kcols : g.M);
+                // the kernel reads whole row blocks of 16 and k steps of 4
+                const int64_t mr = (g.M + 15) / 16 * 16, kr = (kcols + 3) / 4 * 4;
+                const int64_t read = g.transA ? aoff + (mr - 1) * g.lda + kr : aoff + (kr - 1) * g.lda + mr;
+                return aoff >= 0 && last <= pl.opmat_total && g.lda >= (g.transA ? kcols : g.M) &&
+                       read <= pl.opmat_total + pl.opmat_pad;
             };
             if (g.kb == 0) {
                 need(a_ok(g.aoff, g.K), "gemm A");
@@ -1026,6 +1040,7 @@ void Builder::operator_layout() {
     // ---------------- operator table layout: uploaded part, then generated part
     up_n = (int64_t)pl.opmat.size();
     pl.opmat_total = up_n + gen_cursor;
+    pl.opmat_up = up_n;
     for (auto& k : pl.kgen) k.out += up_n;
     pl.stats.opmat_elems = pl.opmat_total;
     pl.stats.opmat_generated = gen_cursor;
@@ -1689,8 +1704,50 @@ void Builder::stages_leaf() {
     merge_sections();
 }
 
+// Packed copies of the operator blocks that the translation GEMMs read (each block once per
+// operand order); their groups then point into the packed table.
+void Builder::pack_operators() {
+    std::map<std::pair<int64_t, int>, int64_t> done;      // (table offset, order) -> packed offset
+    auto packed = [&](int64_t off, int K, const GGroup& g) {
+        auto it = done.find({off, g.transA});
+        if (it != done.end()) {
+            const PackA& p = pl.pack[it->second];
+            if (p.M != g.M || p.K != K || p.lda != g.lda) throw Error("internal: operator block packed in two shapes");
+            return p.dst;
+        }
+        PackA p{};
+        p.src = off; p.dst = pl.pack_total; p.M = g.M; p.K = K; p.lda = g.lda; p.trans = g.transA;
+        pl.pack_total += (int64_t)((K + 7) / 8) * ((g.M + 15) / 16) * 128;
+        done[{off, g.transA}] = (int64_t)pl.pack.size();
+        pl.pack.push_back(p);
+        return p.dst;
+    };
+    std::vector<char> seen(pl.groups.size(), 0);
+    for (Stage& st : pl.stages) {
+        if (st.kind != ST_GEMM || st.prec != PREC_TRANSLATION) continue;
+        for (int t = st.begin; t < st.end; ++t) {
+            if (seen[pl.tiles[t].g]) continue;
+            seen[pl.tiles[t].g] = 1;
+            GGroup& g = pl.groups[pl.tiles[t].g];
+            if (g.soff >= 0) throw Error("internal: row scale on a packed operator");
+            if (g.kb == 0) {
+                g.aoff = packed(g.aoff, g.K, g);
+            } else {
+                for (int h = 0; h < g.K / g.kb; ++h) pl.colA[g.acol0 + h] = packed(pl.colA[g.acol0 + h], g.kb, g);
+            }
+            g.lda = (g.M + 15) / 16;
+            g.transA = 2;
+        }
+        st.trans = 2;
+    }
+}
+
 void Builder::finish(bool want_dump) {
     auto& boxes = tree.boxes;
+    if (prm.pack) pack_operators();
+    for (const GGroup& g : pl.groups)
+        if (g.transA != 2)
+            pl.opmat_pad = std::max(pl.opmat_pad, 16 * (int64_t)g.lda + 16);
     // ---------------- per-stage algorithmic work (per RHS)
     for (auto& st : pl.stages) stage_work(pl, st);
 

@@ -41,6 +41,10 @@ struct HostPlan {
     std::vector<double> px, py, pz;        // leaf-sorted points then LF operator point sets
     std::vector<cpx> opmat;                // uploaded operator tables (prefix of the table)
     int64_t opmat_total = 0;               // uploaded + generated
+    int64_t opmat_up = 0;                  // uploaded part alone
+    std::vector<PackA> pack;               // operator blocks packed at setup (Params::pack)
+    int64_t pack_total = 0;                // elements of the packed table
+    int64_t opmat_pad = 0;                 // zeros behind the table: the GEMM reads whole row blocks and steps
     std::vector<int> grid;                 // FFT grid index tables
     std::vector<double> genpts;            // kernel-generation point table (xyz rows)
     std::vector<KGen> kgen;
