@@ -1518,7 +1518,10 @@ __global__ __launch_bounds__(VL_THREADS) void vlist_acc_kernel(const VTarget* __
 // Eight lanes work on one target: lane l takes frequency l / R1 and the R2 right-hand
 // sides (l % R1) * R2 + q, so the eight lanes read one whole source row per pair (all 32
 // banks) and one tensor value serves R2 complex FMAs.  The accumulated target spectra go
-// to TSPEC in the [rhs][target][(2P)^3] layout of the inverse transform.
+// to TSPEC right-hand side fastest too: the eight lanes of a target write one 128-byte run
+// (with a slab per right-hand side they were pieces of 8 or 16 bytes, written back to HBM as
+// partial lines: V list with its inverse 12.9 -> 8.7 ms at 250k points x 64 RHS, 6.3 -> 4.9 ms at
+// 4M x 8, 3.3 -> 2.2 ms at 250k x 16).
 template <class V> struct VMulti { static constexpr int R2 = 16 / (int)sizeof(V); };   // float2: 2, double2: 1
 
 template <class V, int F, int R1>
@@ -1567,7 +1570,6 @@ __global__ __launch_bounds__(VL_THREADS) void vlist_acc_multi_kernel(const VTarg
     const V* tabl = tab + fl;
     const V* srcl = src + l * R2;
     V* out = bufp<V>(bt, BUF_TSPEC);
-    const int64_t os = bt.stride[BUF_TSPEC];
     for (int sl = 0; sl < NSL; ++sl) {
         const int f0 = fg + sl * F;
         __syncthreads();
@@ -1611,60 +1613,64 @@ __global__ __launch_bounds__(VL_THREADS) void vlist_acc_multi_kernel(const VTarg
 #pragma unroll
                     for (int q = 0; q < R2; ++q) cfma(acc[q], sv[u][q], tv[u]);   // operand order of the 1-RHS kernel
             }
-#pragma unroll
-            for (int q = 0; q < R2; ++q) {
-                const int r = rg + rq + q;
-                if (r < nrhs) out[(int64_t)r * os + (int64_t)(i - v0) * G3 + f0 + fl] = acc[q];
+            V* o = out + ((int64_t)(i - v0) * G3 + f0 + fl) * nrhs + rg + rq;
+            if constexpr (R2 == 2) {
+                typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
+                if (rg + rq + 1 < nrhs) *(f4u*)o = f4u{acc[0].x, acc[0].y, acc[R2 - 1].x, acc[R2 - 1].y};
+                else if (rg + rq < nrhs) o[0] = acc[0];
+            } else {
+                if (rg + rq < nrhs) o[0] = acc[0];
             }
         }
     }
 }
 
 // V list, inverse: one block per target and group of R right-hand sides, the accumulated
-// spectra back to the 6^3 sub-cube (pruned inverse DFT, 1/(2P)^3 scaling) and added into
-// the target's check values.  Each pass runs the R right-hand sides' lines together
-// (R x 144 x lines read straight from the spectra, R x 72 y lines, R x 36 z lines over the
-// block's threads).  LDS: R x 1296 values (41 KB for R = 4 in FP32 or 2 in FP64).
+// spectra (right-hand side fastest, as the source spectra) back to the 6^3 sub-cube (pruned
+// inverse DFT, 1/(2P)^3 scaling) and added into the target's check values.  Each pass runs
+// the R right-hand sides' lines together (R x 144 x lines read straight from the spectra,
+// adjacent lanes on adjacent right-hand sides; R x 72 y lines, R x 36 z lines over the
+// block's threads).  The groups of one target are adjacent items, so they share the spectra's
+// lines in one L2.  LDS: R x 1298 values (41 KB for R = 4 in FP32 or 2 in FP64), each
+// right-hand side's slab padded by one value against the x pass's bank conflicts.
 template <class V, int R>
 __global__ __launch_bounds__(256) void vlist_inv_kernel(const VTarget* __restrict__ vt, const int* __restrict__ grid,
-                                                        int NL, BufTable bt, int v0, int nv, int nrhs) {
+                                                        int NL, BufTable bt, int v0, int nrhs) {
     constexpr int G3 = 1728;
-    __shared__ V A[R][864], B[R][432];
-    const int r0 = blockIdx.y * R, nr = min(R, nrhs - r0);
+    __shared__ V A[R][865], B[R][433];
+    const int groups = (nrhs + R - 1) / R;
+    const int item = xcd_item(blockIdx.x, gridDim.x);
+    const int i = item / groups, r0 = (item - i * groups) * R, nr = min(R, nrhs - r0);
     const int t = threadIdx.x;
-    const int64_t is = bt.stride[BUF_TSPEC], os = bt.stride[BUF_LF_CHK];
-    for (int bi = blockIdx.x; bi < nv; bi += gridDim.x) {
-        const int i = xcd_item(bi, nv);
-        const VTarget tg = vt[v0 + i];
-        const V* in = bufp<V>(bt, BUF_TSPEC) + (int64_t)r0 * is + (int64_t)i * G3;
-        __syncthreads();
-        for (int e = t; e < nr * 144; e += blockDim.x) {   // x lines (ky, kz): 12 inputs -> x' in [6, 12)
-            const int r = e / 144, l = e % 144;
-            dft12_line<V, 12, 6, 0, 6, 1>(in + (int64_t)r * is + 12 * l, 1, A[r] + 6 * l, 1);
-        }
-        __syncthreads();
-        for (int e = t; e < nr * 72; e += blockDim.x) {    // y lines (x', kz): A -> B[kz][y'][x']
-            const int r = e / 72, l = e % 72;
-            dft12_line<V, 12, 6, 0, 6, 1>(A[r] + (l % 6) + 72 * (l / 6), 6, B[r] + (l % 6) + 36 * (l / 6), 6);
-        }
-        __syncthreads();
-        for (int e = t; e < nr * 36; e += blockDim.x) {    // z lines (x', y'): B -> C[z'][y'][x'] (reuses A)
-            const int r = e / 36, l = e % 36;
-            dft12_line<V, 12, 6, 0, 6, 1>(B[r] + l, 36, A[r] + l, 36);
-        }
-        __syncthreads();
-        V* out = bufp<V>(bt, BUF_LF_CHK) + (int64_t)r0 * os + tg.out_off;
-        const typename Real<V>::T coef = (typename Real<V>::T)(1.0 / G3);
-        for (int e = t; e < nr * NL; e += blockDim.x) {
-            const int r = e / NL, k = e % NL;
-            const int g = grid[tg.grid + k];
-            const V v = A[r][(g % 12 - 6) + 6 * ((g / 12) % 12 - 6) + 36 * (g / 144 - 6)];
-            V* o = out + (int64_t)r * os + k;
-            V w = *o;
-            w.x += v.x * coef;
-            w.y += v.y * coef;
-            *o = w;
-        }
+    const int64_t os = bt.stride[BUF_LF_CHK];
+    const VTarget tg = vt[v0 + i];
+    const V* in = bufp<V>(bt, BUF_TSPEC) + (int64_t)i * G3 * nrhs + r0;
+    for (int e = t; e < nr * 144; e += blockDim.x) {   // x lines (ky, kz): 12 inputs -> x' in [6, 12)
+        const int l = e / nr, r = e - l * nr;
+        dft12_line<V, 12, 6, 0, 6, 1>(in + (int64_t)(12 * l) * nrhs + r, nrhs, A[r] + 6 * l, 1);
+    }
+    __syncthreads();
+    for (int e = t; e < nr * 72; e += blockDim.x) {    // y lines (x', kz): A -> B[kz][y'][x']
+        const int r = e / 72, l = e % 72;
+        dft12_line<V, 12, 6, 0, 6, 1>(A[r] + (l % 6) + 72 * (l / 6), 6, B[r] + (l % 6) + 36 * (l / 6), 6);
+    }
+    __syncthreads();
+    for (int e = t; e < nr * 36; e += blockDim.x) {    // z lines (x', y'): B -> C[z'][y'][x'] (reuses A)
+        const int r = e / 36, l = e % 36;
+        dft12_line<V, 12, 6, 0, 6, 1>(B[r] + l, 36, A[r] + l, 36);
+    }
+    __syncthreads();
+    V* out = bufp<V>(bt, BUF_LF_CHK) + (int64_t)r0 * os + tg.out_off;
+    const typename Real<V>::T coef = (typename Real<V>::T)(1.0 / G3);
+    for (int e = t; e < nr * NL; e += blockDim.x) {
+        const int r = e / NL, k = e % NL;
+        const int g = grid[tg.grid + k];
+        const V v = A[r][(g % 12 - 6) + 6 * ((g / 12) % 12 - 6) + 36 * (g / 144 - 6)];
+        V* o = out + (int64_t)r * os + k;
+        V w = *o;
+        w.x += v.x * coef;
+        w.y += v.y * coef;
+        *o = w;
     }
 }
 
@@ -1961,8 +1967,7 @@ hipError_t launch_stage_t(const DevPlan& d, const Stage& s, int nrhs, hipStream_
         }
         {
             constexpr int R = sizeof(V) == 8 ? 4 : 2;      // right-hand sides per block
-            vlist_inv_kernel<V, R><<<dim3(s.stream ? std::min(n, AUX_BLOCKS) : n, (nrhs + R - 1) / R), 256, 0, st>>>(
-                d.vtrg, d.grid, d.NL, d.bt, s.begin, n, nrhs);
+            vlist_inv_kernel<V, R><<<n * ((nrhs + R - 1) / R), 256, 0, st>>>(d.vtrg, d.grid, d.NL, d.bt, s.begin, nrhs);
         }
         break;
     }

@@ -23,6 +23,7 @@ enum Buf : int {
     BUF_SPEC,       // LF V-list source spectra of one level, (2P)^3 each
     BUF_RED,        // HF M2L/L2L contributions of one level, one slot per (target, source)
     BUF_TSPEC,      // LF V-list target spectra of one level, (2P)^3 each, in V-target order
+                    // (BUF_SPEC and BUF_TSPEC: right-hand side fastest, [box][frequency][rhs])
     BUF_NMIR,       // near-field mirror products, one slot per pair evaluated both ways (the
                     // slots into one leaf adjacent, in source-task order)
     BUF_COUNT
