@@ -320,8 +320,9 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         d.grid = c->upload(h.grid);
         const int64_t table = h.opmat_total + h.opmat_pad;
         d.opmat = c->alloc<double2>(table);
-        if (h.opmat_pad > 0)
-            HIPCHK(hipMemset(d.opmat + h.opmat_total, 0, (size_t)h.opmat_pad * sizeof(double2)));
+        // cleared: the setup's products read up to a row block and k step past a block, where
+        // the table may not be written yet, and multiply such k with zeros
+        HIPCHK(hipMemset(d.opmat, 0, (size_t)table * sizeof(double2)));
         if (!h.opmat.empty())
             HIPCHK(hipMemcpy(d.opmat, h.opmat.data(), h.opmat.size() * sizeof(double2), hipMemcpyHostToDevice));
         d.ktasks = c->upload(h.ktasks); d.ksrcs = c->upload(h.ksrcs);
