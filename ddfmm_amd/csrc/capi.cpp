@@ -125,8 +125,8 @@ static void plan_bytes(const HostPlan& h, int precision, int64_t& fixed, int64_t
     const bool mixed = precision == DDFMM_MIXED || precision == DDFMM_MIXED_SPLIT;
     fixed = vbytes(h.px) + vbytes(h.py) + vbytes(h.pz) + 2 * vbytes(h.perm) + vbytes(h.grid) +
             (h.opmat_total + h.opmat_pad) * (int64_t)sizeof(double2) +
-            (mixed ? (h.prm.pack ? h.opmat_up : h.opmat_total) * (int64_t)sizeof(float2) : 0) +
-            h.pack_total * (int64_t)sizeof(float2) +
+            (mixed ? (h.prm.xlat == 1 ? h.opmat_up : h.opmat_total) * (int64_t)sizeof(float2) : 0) +
+            h.pack32_total * (int64_t)sizeof(float2) + h.pack64_total * (int64_t)sizeof(double2) +
             (precision == DDFMM_MIXED_SPLIT ? h.opmat_total * 16 : 0) +
             vbytes(h.ktasks) + vbytes(h.ksrcs) + vbytes(h.groups) + vbytes(h.tiles) + vbytes(h.colB) +
             vbytes(h.colC) + vbytes(h.colA) + vbytes(h.fsrc) + vbytes(h.vtrg) + vbytes(h.vchunk) +
@@ -135,7 +135,7 @@ static void plan_bytes(const HostPlan& h, int precision, int64_t& fixed, int64_t
     per_rhs = 2 * h.N * (int64_t)sizeof(double2);
     for (int b = 0; b < BUF_COUNT; ++b) per_rhs += h.bufsize[b] * esz;
     for (int b = 0; b < BUF_COUNT; ++b) fixed += h.bufsize[b] > 0 ? BUF_SLACK * esz : 0;
-    transient = std::max(vbytes(h.genpts) + vbytes(h.kgen), vbytes(h.pack));
+    transient = std::max(vbytes(h.genpts) + vbytes(h.kgen), std::max(vbytes(h.pack32), vbytes(h.pack64)));
 }
 
 // The kernel-apply flavour is fixed per context (each right-hand side then has the same
@@ -267,7 +267,7 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         q.numC = p->numC; q.ktype = p->kernel;
         q.fuse_solves = p->precision != DDFMM_FP64;
         q.nrhs_max = p->nrhs_max;
-        q.pack = p->precision == DDFMM_MIXED;
+        q.xlat = p->precision == DDFMM_MIXED ? 1 : p->precision == DDFMM_MIXED_SPLIT ? 2 : 0;
         // the matrix-core kernel apply (mixed modes, four or more right-hand sides)
         // evaluates near-field leaf pairs of a small leaf once for both directions; with
         // leaves of up to 128 points most pairs qualify (with larger leaves few do, and the
@@ -354,24 +354,28 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
             HIPCHK(hipStreamSynchronize(c->stream));
         }
         if (d.mixed) {
-            const int64_t n32 = h.prm.pack ? h.opmat_up : h.opmat_total;
+            const int64_t n32 = h.prm.xlat == 1 ? h.opmat_up : h.opmat_total;
             d.opmat32 = c->alloc<float2>(n32);
             HIPCHK(launch_to_f32(d.opmat, d.opmat32, n32, c->stream));
-            if (!h.pack.empty()) {
-                d.oppack = c->alloc<float2>(h.pack_total);
-                PackA* jobs = nullptr;
-                HIPCHK(hipMalloc(&jobs, h.pack.size() * sizeof(PackA)));
-                HIPCHK(hipMemcpy(jobs, h.pack.data(), h.pack.size() * sizeof(PackA), hipMemcpyHostToDevice));
-                // three products (e^{ikr}/r) take k in pairs, four keep the stored order
-                HIPCHK(launch_pack(jobs, (int)h.pack.size(), d.opmat, d.oppack, d.ktype == 0, c->stream));
-                HIPCHK(hipStreamSynchronize(c->stream));
-                HIPCHK(hipFree(jobs));
-            }
             if (c->precision == DDFMM_MIXED_SPLIT) {    // translations as split-BF16 products
                 d.opmatbf = (void*)c->alloc<double2>(h.opmat_total);
                 HIPCHK(launch_to_bf16s(d.opmat, d.opmatbf, h.opmat_total, c->stream));
             }
             HIPCHK(hipStreamSynchronize(c->stream));
+        }
+        // the GEMMs' operators in lane order (three products, e^{ikr}/r in FP32, take k in pairs)
+        d.oppack = c->alloc<float2>(h.pack32_total);
+        d.oppack64 = c->alloc<double2>(h.pack64_total);
+        for (int f32 = 0; f32 < 2; ++f32) {
+            const std::vector<PackA>& pk = f32 ? h.pack32 : h.pack64;
+            if (pk.empty()) continue;
+            PackA* jobs = nullptr;
+            HIPCHK(hipMalloc(&jobs, pk.size() * sizeof(PackA)));
+            HIPCHK(hipMemcpy(jobs, pk.data(), pk.size() * sizeof(PackA), hipMemcpyHostToDevice));
+            HIPCHK(launch_pack(jobs, (int)pk.size(), d.opmat, f32 ? (void*)d.oppack : (void*)d.oppack64, f32,
+                               d.ktype == 0, c->stream));
+            HIPCHK(hipStreamSynchronize(c->stream));
+            HIPCHK(hipFree(jobs));
         }
         // work buffers, after the setup-time tables are gone
         for (int b = 0; b < BUF_COUNT; ++b) {
@@ -385,7 +389,8 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         std::vector<cpx>().swap(h.opmat);
         std::vector<double>().swap(h.genpts);
         std::vector<KGen>().swap(h.kgen);
-        std::vector<PackA>().swap(h.pack);
+        std::vector<PackA>().swap(h.pack32);
+        std::vector<PackA>().swap(h.pack64);
         c->ready = true;
     } catch (const HipFail& e) {
         c->release();

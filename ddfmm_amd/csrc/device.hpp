@@ -32,7 +32,8 @@ struct DevPlan {
     int* grid = nullptr;
     double2* opmat = nullptr;
     float2* opmat32 = nullptr;     // FP32 copy of the operator table (mixed modes; MIXED: its uploaded part)
-    float2* oppack = nullptr;      // packed FP32 operator blocks of the translation GEMMs (MIXED)
+    float2* oppack = nullptr;      // packed operator blocks of the GEMMs: FP32 (MIXED translations)
+    double2* oppack64 = nullptr;   // and FP64 (every other GEMM but the split-BF16 ones)
     void* opmatbf = nullptr;       // split-BF16 copy (16 bytes per entry; mixed-split mode)
     KTask* ktasks = nullptr;
     KSrc* ksrcs = nullptr;
@@ -71,7 +72,7 @@ hipError_t launch_direct(const double* trg, int M, const double* src, int Ns, co
 hipError_t direct_static_scratch(double2** out);
 hipError_t launch_kmatrix(const double* trg, int M, const double* src, int Ns, void* out, int ktype, int f32,
                           hipStream_t st);
-hipError_t launch_pack(const PackA* jobs, int njobs, const double2* opmat, float2* out, int pair, hipStream_t st);
+hipError_t launch_pack(const PackA* jobs, int njobs, const double2* opmat, void* out, int f32, int pair, hipStream_t st);
 hipError_t launch_to_f32(const double2* in, float2* out, int64_t n, hipStream_t st);
 hipError_t launch_to_bf16s(const double2* in, void* out, int64_t n, hipStream_t st);
 

@@ -704,24 +704,26 @@ __device__ __forceinline__ CPair load_pair(const float2* p) {
     return {{make_float2(r.x, r.y), make_float2(r.z, r.w)}};
 }
 
-// A's form: as stored (column-major blocks), transposed as stored, or packed (FP32, PackA in
-// plan.hpp) in the order the lanes take it.
-enum GemmA : int { GEMM_A = 0, GEMM_AT = 1, GEMM_APACK = 2 };
+// Units (8 k in FP32, 4 in FP64) per pipeline step: short tiles run few MFMAs per unit, so
+// they load further ahead.  U2U of 6k points in FP64 (858 waves of one row block) 0.123 -> 0.104
+// ms, of 60k 0.39 -> 0.35; twice as many units at one and two row blocks: 0.103 and 0.37.
+constexpr int gemm_units(int mb, int cb) { return cb > 1 || mb > 3 ? 1 : mb > 1 ? 2 : 4; }
 
-template <class TA, class V, class R, int MB, int CB, int AF, bool G3M>
+// PACK: A packed (PackA in plan.hpp) in the order the lanes take it; else as stored, column
+// major (the setup's products on the operator table itself).
+template <class TA, class V, class R, int MB, int CB, bool PACK, bool G3M>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(
     const GGroup* __restrict__ groups, const GTile* __restrict__ tiles,
     const int64_t* __restrict__ colB, const int64_t* __restrict__ colC, const int64_t* __restrict__ colA,
-    const TA* __restrict__ opm, BufTable bt, int tile0, int nr) {
+    const TA* __restrict__ opm, const double2* __restrict__ scl, BufTable bt, int tile0, int nr) {
     using M = Mfma<R>;
     using T = typename Real<V>::T;
     constexpr int TN = GEMM_TN * CB;
-    constexpr bool TRANS = AF == GEMM_AT, PACK = AF == GEMM_APACK;
-    constexpr int KQ = PACK ? 2 : 1, KS = 4 * KQ;      // k steps and k per pipeline step
-    // k order of a pipeline step: with three products lane group lk takes k = 2 lk + q in k
-    // step q (one 16-byte load of B; a last step of at most 4 k runs k = lk alone), with four
-    // k = lk + 4 q
-    constexpr bool PAIR = PACK && G3M;
+    constexpr int UQ = sizeof(R) == 4 ? 2 : 1, UK = 4 * UQ;          // k steps and k per unit
+    constexpr int NU = gemm_units(MB, CB), KQ = NU * UQ, KS = NU * UK;   // per pipeline step
+    // k order of a unit: with three products lane group lk takes k = 2 lk + q in k step q (one
+    // 16-byte load of B; a last unit of at most 4 k runs k = lk alone), with four k = lk + 4 q
+    constexpr bool PAIR = G3M;
     // columns are (box, rhs) pairs, rhs fastest: column n is box n / nr of the group in
     // right-hand side n % nr (that rhs slab of the buffer).  A planned tile (GEMM_TN boxes)
     // becomes ceil(nr / CB) launched tiles of TN such columns; waves past its boxes or the
@@ -772,12 +774,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         }
         wave_lds_order();
     }
+    // A elements of this lane within a unit, per row block and per unit
+    constexpr unsigned ROWS = PACK ? 64 * UQ : 16;
     const unsigned lda = g.lda;
-    unsigned ao[TRANS ? MB : 1];                        // this lane's A offset (of each row block)
-#pragma unroll
-    for (int a = 0; a < (TRANS ? MB : 1); ++a)
-        ao[a] = PACK ? 2 * lane : TRANS ? (16 * a + li) * lda + lk : lk * lda + li;
-    const unsigned kstep = PACK ? 128 * lda : TRANS ? KS : KS * lda;    // A elements per pipeline step
+    const unsigned ao = PACK ? UQ * lane : lk * lda + li, ustep = PACK ? ROWS * lda : UK * lda;
 
     // G3M (FP32 contexts of the e^{ikr}/r kernel): three real products per complex one,
     // summed over k apart: k1 = (Ar + Ai) Br, k2 = Ar (Bi - Br), k3 = Ai (Br + Bi); Re C =
@@ -805,7 +805,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         int kl;                    // k left in the segment
         bool fix;                  // some entry of b must be zeroed
     };
-    // loader: the current segment's A position and columns, and the k range of the step
+    // loader: the current segment's A block and columns, and the k range of the step
+    const int ktop = (kb - 1) / UK * UK;       // first k of a segment's last unit
     const TA* Ap = nullptr;
     const V* Bp[CB];
     bool pres[CB];
@@ -814,7 +815,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     auto segment = [&]() {
         const int h = __builtin_ctz(act);
         act &= act - 1;
-        Ap = opm + (g.kb ? colA[g.acol0 + h] : g.aoff) + (TRANS ? (int64_t)tl.m0 * lda : PACK ? 8 * tl.m0 : tl.m0);
+        Ap = opm + (g.kb ? colA[g.acol0 + h] : g.aoff) + (PACK ? ROWS / 16 * tl.m0 : tl.m0);
         k0 = 0;
         kl = kb;
         bool all = true;
@@ -831,7 +832,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         if (kl > KS) {
             k0 += KS;
             kl -= KS;
-            Ap += kstep;
             return true;
         }
         if (!act) return false;
@@ -841,34 +841,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     // The loads of a step are unconditional and in one block (past the last step they repeat
     // it), so that the waits before their use count the next step's loads as outstanding.
     auto fetch = [&](Step& s) {
-        if constexpr (PAIR) {
-            // the pair's second entry is at most kb (BUF_SLACK)
-            const int k = min(k0 + (kl <= 4 ? lk : 2 * lk), kb - 1);
 #pragma unroll
-            for (int c = 0; c < CB; ++c) {
-                const CPair b = load_pair(Bp[c] + k);
-                s.b[0][c] = b.e[0];
-                s.b[KQ - 1][c] = b.e[1];
+        for (int u = 0; u < NU; ++u) {
+            const int ku = NU == 1 ? k0 : min(k0 + u * UK, ktop);
+            if constexpr (PAIR) {
+                // the pair's second entry is at most kb (BUF_SLACK)
+                const int k = min(ku + (kb - ku <= 4 ? lk : 2 * lk), kb - 1);
+#pragma unroll
+                for (int c = 0; c < CB; ++c) {
+                    const CPair b = load_pair(Bp[c] + k);
+                    s.b[u * UQ][c] = b.e[0];
+                    s.b[u * UQ + UQ - 1][c] = b.e[1];
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < UQ; ++q) {
+                    const int k = min(ku + 4 * q + lk, kb - 1);
+#pragma unroll
+                    for (int c = 0; c < CB; ++c) s.b[u * UQ + q][c] = Bp[c][k];
+                }
             }
-        } else {
-#pragma unroll
-            for (int q = 0; q < KQ; ++q) {
-                const int k = min(k0 + 4 * q + lk, kb - 1);
-#pragma unroll
-                for (int c = 0; c < CB; ++c) s.b[q][c] = Bp[c][k];
-            }
-        }
-        if constexpr (PACK) {
+            const TA* ap = Ap + (unsigned)(ku / UK) * ustep + ao;
 #pragma unroll
             for (int a = 0; a < MB; ++a) {
-                const float4 v = *(const float4*)(Ap + 128 * a + ao[0]);
-                s.a[0][a] = make_float2(v.x, v.y);
-                s.a[KQ - 1][a] = make_float2(v.z, v.w);
+                if constexpr (PACK && sizeof(R) == 4) {
+                    const float4 v = *(const float4*)(ap + ROWS * a);
+                    s.a[u * UQ][a] = make_float2(v.x, v.y);
+                    s.a[u * UQ + UQ - 1][a] = make_float2(v.z, v.w);
+                } else {
+                    s.a[u * UQ][a] = ap[ROWS * a];
+                }
             }
-        } else {
-            const TA* ap = Ap + ao[0];
-#pragma unroll
-            for (int a = 0; a < MB; ++a) s.a[0][a] = TRANS ? Ap[ao[TRANS ? a : 0]] : ap[16 * a];
         }
 #pragma unroll
         for (int c = 0; c < CB; ++c) s.p[c] = pres[c];
@@ -880,10 +883,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     auto compute = [&](Step& s) {
         if (s.fix) {
 #pragma unroll
-            for (int q = 0; q < KQ; ++q)
+            for (int q = 0; q < KQ; ++q) {
+                const int kl = s.kl - q / UQ * UK;     // k left from the unit's first
+                const int kq = PAIR && kl > 4 ? 2 * lk + q % UQ : 4 * (q % UQ) + lk;
 #pragma unroll
                 for (int c = 0; c < CB; ++c)
-                    if (!s.p[c] || (PAIR && s.kl > 4 ? 2 * lk + q : 4 * q + lk) >= s.kl) s.b[q][c] = mk<V>(0, 0);
+                    if (!s.p[c] || kq >= kl) s.b[q][c] = mk<V>(0, 0);
+            }
         }
 #pragma unroll
         for (int q = 0; q < KQ; ++q) {
@@ -949,7 +955,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
             if constexpr (sizeof(R) == 4) {      // four adjacent rows: two 16-byte stores
                 typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
                 const int m = tl.m0 + 16 * a + 4 * lk;
-                if (g.soff < 0 && g.mode == 0 && m + 3 < g.M) {
+                if (g.mode == 0 && m + 3 < g.M) {
                     f4u lo = {re[0], im[0], re[1], im[1]}, hi = {re[2], im[2], re[3], im[3]};
                     *(f4u*)(Cc + m) = lo;
                     *(f4u*)(Cc + m + 2) = hi;
@@ -961,12 +967,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
                 const int m = tl.m0 + 16 * a + M::row(lk, v);
                 if (m >= g.M) continue;
                 R x = re[v], y = im[v];
-                if (g.soff >= 0) {
-                    const TA s = opm[g.soff + m];
-                    const R sr = (R)s.x, si = (R)s.y;
-                    const R t = x * sr - y * si;
-                    y = x * si + y * sr;
-                    x = t;
+                if constexpr (sizeof(R) == 8) {        // row scales: FP64 groups only
+                    if (g.soff >= 0) {
+                        const double2 s = scl[g.soff + m];
+                        const R t = x * s.x - y * s.y;
+                        y = x * s.y + y * s.x;
+                        x = t;
+                    }
                 }
                 if (g.mode == 0) {
                     Cc[m] = mk<V>(x, y);
@@ -981,27 +988,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     }
 }
 
-template <class TA, class V, class R, int CB, int AF, bool G3M>
-void launch_gemm_form(int mb, int n, int nrhs, hipStream_t st, const DevPlan& d, const TA* opm, int t0) {
-    const dim3 grid(n * ((nrhs + CB - 1) / CB), 1);
-#define DDFMM_GEMM_MB(X)                                                                                          \
-    case X:                                                                                                       \
-        gemm_kernel<TA, V, R, X, CB, AF, G3M><<<grid, 256, 0, st>>>(d.groups, d.tiles, d.colB, d.colC, d.colA,   \
-                                                                    opm, d.bt, t0, nrhs);                        \
+template <class TA, class V, class R, int CB, bool PACK, bool G3M>
+void launch_gemm_form(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d, const TA* opm) {
+    const dim3 grid((s.end - s.begin) * ((nrhs + CB - 1) / CB), 1);
+#define DDFMM_GEMM_MB(X)                                                                                            \
+    case X:                                                                                                         \
+        gemm_kernel<TA, V, R, X, CB, PACK, G3M><<<grid, 256, 0, st>>>(d.groups, d.tiles, d.colB, d.colC, d.colA,   \
+                                                                      opm, d.opmat, d.bt, s.begin, nrhs);          \
         break;
-    switch (mb) {
+    switch (s.mb) {
         DDFMM_GEMM_MB(1) DDFMM_GEMM_MB(2) DDFMM_GEMM_MB(3) DDFMM_GEMM_MB(4) DDFMM_GEMM_MB(5)
         DDFMM_GEMM_MB(6) DDFMM_GEMM_MB(7)
     }
 #undef DDFMM_GEMM_MB
-}
-
-// FP64 products on operators as stored.
-template <class V>
-void launch_gemm64(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
-    const int n = s.end - s.begin;
-    if (s.trans) launch_gemm_form<double2, V, double, 1, GEMM_AT, false>(s.mb, n, nrhs, st, d, d.opmat, s.begin);
-    else launch_gemm_form<double2, V, double, 1, GEMM_A, false>(s.mb, n, nrhs, st, d, d.opmat, s.begin);
 }
 
 // FP32 products on packed operators.  Two column blocks per wave (CB = 2) halve the operator
@@ -1011,27 +1010,27 @@ void launch_gemm64(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
 // U2U 17.3 -> 18.1 ms) and the launch still has four blocks per CU.
 template <bool G3M>
 void launch_gemm32(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
-    const int n = s.end - s.begin;
-    if (nrhs >= 32 && !s.kblocked && (int64_t)n * nrhs / 2 >= 1024 && s.mb < GEMM_MB)
-        launch_gemm_form<float2, float2, float, 2, GEMM_APACK, G3M>(s.mb, n, nrhs, st, d, d.oppack, s.begin);
+    if (nrhs >= 32 && !s.kblocked && (int64_t)(s.end - s.begin) * nrhs / 2 >= 1024 && s.mb < GEMM_MB)
+        launch_gemm_form<float2, float2, float, 2, true, G3M>(s, nrhs, st, d, d.oppack);
     else
-        launch_gemm_form<float2, float2, float, 1, GEMM_APACK, G3M>(s.mb, n, nrhs, st, d, d.oppack, s.begin);
+        launch_gemm_form<float2, float2, float, 1, true, G3M>(s, nrhs, st, d, d.oppack);
 }
 
-// One packed operator block per job (PackA): rows in blocks of 16 and k in steps of 8, zeros
-// past the block's edges.
+// One packed operator block per job (PackA): zeros past the block's edges.
+template <class T>
 __global__ __launch_bounds__(256) void pack_kernel(const PackA* __restrict__ jobs, const double2* __restrict__ opmat,
-                                                   float2* __restrict__ out, int pair) {
+                                                   T* __restrict__ out, int pair) {
+    constexpr int UQ = 16 / (int)sizeof(T), UK = 4 * UQ;
     const PackA p = jobs[blockIdx.x];
-    const int nrb = (p.M + 15) / 16, nk = (p.K + 7) / 8;
-    for (int e = threadIdx.x; e < nrb * nk * 128; e += 256) {
-        const int q = e & 1, lane = (e >> 1) & 63, rb = (e >> 7) % nrb, o = (e >> 7) / nrb;
+    const int nrb = (p.M + 15) / 16, nk = (p.K + UK - 1) / UK;
+    for (int e = threadIdx.x; e < nrb * nk * 64 * UQ; e += 256) {
+        const int q = e % UQ, lane = e / UQ & 63, rb = e / (64 * UQ) % nrb, o = e / (64 * UQ) / nrb;
         const int m = 16 * rb + (lane & 15), lk = lane >> 4;
-        const int k = 8 * o + (pair && p.K - 8 * o > 4 ? 2 * lk + q : lk + 4 * q);
-        float2 v = make_float2(0.f, 0.f);
+        const int k = UK * o + (pair && p.K - UK * o > 4 ? 2 * lk + q : lk + 4 * q);
+        T v = mk<T>(0, 0);
         if (m < p.M && k < p.K) {
             const double2 a = opmat[p.src + (p.trans ? k + (int64_t)m * p.lda : m + (int64_t)k * p.lda)];
-            v = make_float2((float)a.x, (float)a.y);
+            v = mk<T>(a.x, a.y);
         }
         out[p.dst + e] = v;
     }
@@ -1974,7 +1973,7 @@ hipError_t launch_stage_t(const DevPlan& d, const Stage& s, int nrhs, hipStream_
     case ST_GEMM:
         if (s.mb < 1 || s.mb > GEMM_MB) return hipErrorInvalidValue;
         if (d.mixed && s.prec == PREC_SOLVE)
-            launch_gemm64<float2>(s, nrhs, st, d);
+            launch_gemm_form<double2, float2, double, 1, true, false>(s, nrhs, st, d, d.oppack64);
         else if (d.mixed && d.opmatbf)
             launch_gemm_bf16s(s.mb, n, nrhs, st, d, s.begin);
         else if (d.mixed && d.ktype == 0)    // e^{ikr}/r: three real products per complex one
@@ -1982,7 +1981,7 @@ hipError_t launch_stage_t(const DevPlan& d, const Stage& s, int nrhs, hipStream_
         else if (d.mixed)
             launch_gemm32<false>(s, nrhs, st, d);
         else
-            launch_gemm64<double2>(s, nrhs, st, d);
+            launch_gemm_form<double2, double2, double, 1, true, false>(s, nrhs, st, d, d.oppack64);
         break;
     case ST_FFTFWD:
         if (d.P != 6) return hipErrorInvalidValue;
@@ -2054,7 +2053,7 @@ hipError_t launch_stage(const DevPlan& d, const Stage& s, int nrhs, hipStream_t 
 
 hipError_t launch_setup_gemm(const DevPlan& d, const Stage& s, hipStream_t st) {
     if (s.kind != ST_GEMM || s.mb < 1 || s.mb > GEMM_MB) return hipErrorInvalidValue;
-    launch_gemm64<double2>(s, 1, st, d);
+    launch_gemm_form<double2, double2, double, 1, false, false>(s, 1, st, d, d.opmat);
     return hipGetLastError();
 }
 
@@ -2066,9 +2065,12 @@ hipError_t launch_kgen(const KGen* jobs, int njobs, const double* gp, double2* o
     return hipGetLastError();
 }
 
-hipError_t launch_pack(const PackA* jobs, int njobs, const double2* opmat, float2* out, int pair, hipStream_t st) {
-    for (int j0 = 0; j0 < njobs; j0 += 65536)
-        pack_kernel<<<std::min(65536, njobs - j0), 256, 0, st>>>(jobs + j0, opmat, out, pair);
+hipError_t launch_pack(const PackA* jobs, int njobs, const double2* opmat, void* out, int f32, int pair, hipStream_t st) {
+    for (int j0 = 0; j0 < njobs; j0 += 65536) {
+        const int n = std::min(65536, njobs - j0);
+        if (f32) pack_kernel<float2><<<n, 256, 0, st>>>(jobs + j0, opmat, (float2*)out, pair);
+        else pack_kernel<double2><<<n, 256, 0, st>>>(jobs + j0, opmat, (double2*)out, 0);
+    }
     return hipGetLastError();
 }
 

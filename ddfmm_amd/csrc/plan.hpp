@@ -70,7 +70,7 @@ struct KTask {
 struct GGroup {
     int64_t aoff;   // A offset in the operator table
     int64_t soff;   // row scale (length M) offset, or -1
-    int M, K, lda, transA;      // transA: 0 A[m + k lda], 1 A[k + m lda], 2 packed (PackA)
+    int M, K, lda, transA;      // transA: 0 A[m + k lda], 1 A[k + m lda], 2 / 3 packed FP32 / FP64
     int bbuf, cbuf;
     int ncols, col0;
     int mode;       // 0 store, 1 add
@@ -85,11 +85,12 @@ struct GTile {
 };
 constexpr int GEMM_MB = 7;      // rows per tile <= 112
 constexpr int GEMM_TN = 64;     // columns per tile (16 per wave)
-// The FP32 GEMM's operator blocks, packed at setup in the order its lanes take them: per 8 k
-// and 16 rows, lane li + 16 lk holds row li at the two k of its lane group lk, adjacent
-// (pair: k = 2 lk, 2 lk + 1, unless at most 4 k are left; else lk, lk + 4), so that a wave reads a row block's 8 k by one
-// contiguous 1 KiB load.  8-k steps outermost, then row blocks; zeros past M and K.  A
-// packed group's aoff / colA entries point to its blocks and its lda is their row blocks.
+// The GEMM's operator blocks, packed at setup in the order its lanes take them, so that a
+// wave reads a row block's unit of k (8 in FP32, 4 in FP64) by one contiguous 1 KiB load:
+// lane li + 16 lk holds row li at the unit's k of its lane group lk (FP64: lk; FP32: two
+// adjacent entries, k = 2 lk and 2 lk + 1 with three products, unless at most 4 k are left, else
+// lk and lk + 4).  Units outermost, then row blocks of 16; zeros past M and K.  A packed
+// group's aoff / colA entries point to its blocks and its lda is their row blocks.
 struct PackA {
     int64_t src, dst;           // first element in the operator table / in the packed table
     int M, K, lda, trans;       // the block as stored
@@ -181,7 +182,7 @@ struct Stage {
     int mb;             // ST_GEMM: row blocks of every tile in the range (one kernel instance);
                         // ST_KAPPLY: 1 when sources carry mirror slots (KSrc::moff)
     int lstage;         // ST_GEMM: logical stage (all tile heights of one planned GEMM stage), else -1
-    int trans;          // ST_GEMM: transA of every group in the range (one kernel instance)
+    int trans;          // ST_GEMM: transA of every group in the range
     int kblocked;       // ST_GEMM: the groups' K is blocked (GGroup::kb > 0)
     double exec;        // ST_GEMM: MFMA flops per RHS the kernel executes (padding included)
     char name[24];

@@ -210,6 +210,10 @@ struct Builder {
         pl.opmat.insert(pl.opmat.end(), m.a.begin(), m.a.end());
         return off;
     }
+    static int64_t pack_elems(bool f32, int M, int K) {    // of a packed M x K block
+        const int64_t nrb = (M + 15) / 16;
+        return f32 ? (K + 7) / 8 * nrb * 128 : (K + 3) / 4 * nrb * 64;
+    }
     int64_t genpts(const std::vector<double>& xyz) {
         int64_t off = (int64_t)pl.genpts.size() / 3;
         pl.genpts.insert(pl.genpts.end(), xyz.begin(), xyz.end());
@@ -553,7 +557,7 @@ struct Builder {
             for (int t = st.begin; t < st.end; ++t) {
                 need(pl.tiles[t].mb == st.mb, "setup tile height");
                 const GGroup& g = pl.groups[pl.tiles[t].g];
-                need(g.transA == st.trans, "setup operand order");
+                need(g.transA == 0 && st.trans == 0, "setup operand order");
                 need(g.bbuf == BUF_OPMAT && g.cbuf == BUF_OPMAT, "setup buffers");
             }
         }
@@ -566,12 +570,14 @@ struct Builder {
             }
             if (g.soff >= 0) need(g.soff + g.M <= pl.opmat_total, "gemm row scale");
             auto a_ok = [&](int64_t aoff, int kcols) {
-                if (g.transA == 2)
-                    return aoff >= 0 && aoff % 128 == 0 && g.lda == (g.M + 15) / 16 &&
-                           aoff + (int64_t)((kcols + 7) / 8) * g.lda * 128 <= pl.pack_total;
+                if (g.transA >= 2) {
+                    const bool f32 = g.transA == 2;
+                    return aoff >= 0 && aoff % 64 == 0 && g.lda == (g.M + 15) / 16 &&
+                           aoff + pack_elems(f32, g.M, kcols) <= (f32 ? pl.pack32_total : pl.pack64_total);
+                }
                 const int64_t last = g.transA ? aoff + (int64_t)(g.M - 1) * g.lda + kcols
                                               : aoff + (int64_t)(kcols - 1) * g.lda + g.M;
-                // the kernel reads whole row blocks of 16 and k steps of 4
+                // the kernel reads whole row blocks of 16 and units of 4 k
                 const int64_t mr = (g.M + 15) / 16 * 16, kr = (kcols + 3) / 4 * 4;
                 const int64_t read = g.transA ? aoff + (mr - 1) * g.lda + kr : aoff + (kr - 1) * g.lda + mr;
                 return aoff >= 0 && last <= pl.opmat_total && g.lda >= (g.transA ? kcols : g.M) &&
@@ -1704,49 +1710,53 @@ void Builder::stages_leaf() {
     merge_sections();
 }
 
-// Packed copies of the operator blocks that the translation GEMMs read (each block once per
-// operand order); their groups then point into the packed table.
+// Packed copies of the operator blocks that the evaluation's GEMMs read (each block once per
+// table and operand order); their groups then point into the packed tables.
 void Builder::pack_operators() {
-    std::map<std::pair<int64_t, int>, int64_t> done;      // (table offset, order) -> packed offset
-    auto packed = [&](int64_t off, int K, const GGroup& g) {
-        auto it = done.find({off, g.transA});
-        if (it != done.end()) {
-            const PackA& p = pl.pack[it->second];
+    std::map<std::pair<int64_t, int>, int> done[2];       // FP32, FP64: (table offset, order) -> job
+    auto packed = [&](bool f32, int64_t off, int K, const GGroup& g) {
+        std::vector<PackA>& jobs = f32 ? pl.pack32 : pl.pack64;
+        int64_t& total = f32 ? pl.pack32_total : pl.pack64_total;
+        auto it = done[f32].find({off, g.transA});
+        if (it != done[f32].end()) {
+            const PackA& p = jobs[it->second];
             if (p.M != g.M || p.K != K || p.lda != g.lda) throw Error("internal: operator block packed in two shapes");
             return p.dst;
         }
         PackA p{};
-        p.src = off; p.dst = pl.pack_total; p.M = g.M; p.K = K; p.lda = g.lda; p.trans = g.transA;
-        pl.pack_total += (int64_t)((K + 7) / 8) * ((g.M + 15) / 16) * 128;
-        done[{off, g.transA}] = (int64_t)pl.pack.size();
-        pl.pack.push_back(p);
+        p.src = off; p.dst = total; p.M = g.M; p.K = K; p.lda = g.lda; p.trans = g.transA;
+        total += pack_elems(f32, g.M, K);
+        done[f32][{off, g.transA}] = (int)jobs.size();
+        jobs.push_back(p);
         return p.dst;
     };
     std::vector<char> seen(pl.groups.size(), 0);
     for (Stage& st : pl.stages) {
-        if (st.kind != ST_GEMM || st.prec != PREC_TRANSLATION) continue;
+        if (st.kind != ST_GEMM || (st.prec == PREC_TRANSLATION && prm.xlat == 2)) continue;
+        const bool f32 = st.prec == PREC_TRANSLATION && prm.xlat == 1;
         for (int t = st.begin; t < st.end; ++t) {
             if (seen[pl.tiles[t].g]) continue;
             seen[pl.tiles[t].g] = 1;
             GGroup& g = pl.groups[pl.tiles[t].g];
-            if (g.soff >= 0) throw Error("internal: row scale on a packed operator");
+            if (f32 && g.soff >= 0) throw Error("internal: row scale on an FP32 operator");
             if (g.kb == 0) {
-                g.aoff = packed(g.aoff, g.K, g);
+                g.aoff = packed(f32, g.aoff, g.K, g);
             } else {
-                for (int h = 0; h < g.K / g.kb; ++h) pl.colA[g.acol0 + h] = packed(pl.colA[g.acol0 + h], g.kb, g);
+                for (int h = 0; h < g.K / g.kb; ++h)
+                    pl.colA[g.acol0 + h] = packed(f32, pl.colA[g.acol0 + h], g.kb, g);
             }
             g.lda = (g.M + 15) / 16;
-            g.transA = 2;
+            g.transA = f32 ? 2 : 3;
         }
-        st.trans = 2;
+        st.trans = f32 ? 2 : 3;
     }
 }
 
 void Builder::finish(bool want_dump) {
     auto& boxes = tree.boxes;
-    if (prm.pack) pack_operators();
+    pack_operators();
     for (const GGroup& g : pl.groups)
-        if (g.transA != 2)
+        if (g.transA < 2)
             pl.opmat_pad = std::max(pl.opmat_pad, 16 * (int64_t)g.lda + 16);
     // ---------------- per-stage algorithmic work (per RHS)
     for (auto& st : pl.stages) stage_work(pl, st);

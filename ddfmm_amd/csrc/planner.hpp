@@ -42,9 +42,9 @@ struct HostPlan {
     std::vector<cpx> opmat;                // uploaded operator tables (prefix of the table)
     int64_t opmat_total = 0;               // uploaded + generated
     int64_t opmat_up = 0;                  // uploaded part alone
-    std::vector<PackA> pack;               // operator blocks packed at setup (Params::pack)
-    int64_t pack_total = 0;                // elements of the packed table
-    int64_t opmat_pad = 0;                 // zeros behind the table: the GEMM reads whole row blocks and steps
+    std::vector<PackA> pack32, pack64;     // operator blocks packed at setup, per table
+    int64_t pack32_total = 0, pack64_total = 0;
+    int64_t opmat_pad = 0;                 // zeros behind the table: the setup GEMMs read whole row blocks and units
     std::vector<int> grid;                 // FFT grid index tables
     std::vector<double> genpts;            // kernel-generation point table (xyz rows)
     std::vector<KGen> kgen;
