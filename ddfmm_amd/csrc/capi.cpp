@@ -126,7 +126,7 @@ static void plan_bytes(const HostPlan& h, int precision, int64_t& fixed, int64_t
     fixed = vbytes(h.px) + vbytes(h.py) + vbytes(h.pz) + 2 * vbytes(h.perm) + vbytes(h.grid) +
             (h.opmat_total + h.opmat_pad) * (int64_t)sizeof(double2) +
             (mixed ? (h.prm.xlat == 1 ? h.opmat_up : h.opmat_total) * (int64_t)sizeof(float2) : 0) +
-            h.pack32_total * (int64_t)sizeof(float2) + h.pack64_total * (int64_t)sizeof(double2) +
+            h.pack32_total * (int64_t)sizeof(float2) + (h.pack64_total + h.zeros) * (int64_t)sizeof(double2) +
             (precision == DDFMM_MIXED_SPLIT ? h.opmat_total * 16 : 0) +
             vbytes(h.ktasks) + vbytes(h.ksrcs) + vbytes(h.groups) + vbytes(h.tiles) + vbytes(h.colB) +
             vbytes(h.colC) + vbytes(h.colA) + vbytes(h.fsrc) + vbytes(h.vtrg) + vbytes(h.vchunk) +
@@ -323,6 +323,8 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         // cleared: the setup's products read up to a row block and k step past a block, where
         // the table may not be written yet, and multiply such k with zeros
         HIPCHK(hipMemset(d.opmat, 0, (size_t)table * sizeof(double2)));
+        d.zeros = c->alloc<double2>(h.zeros);
+        HIPCHK(hipMemset(d.zeros, 0, (size_t)h.zeros * sizeof(double2)));
         if (!h.opmat.empty())
             HIPCHK(hipMemcpy(d.opmat, h.opmat.data(), h.opmat.size() * sizeof(double2), hipMemcpyHostToDevice));
         d.ktasks = c->upload(h.ktasks); d.ksrcs = c->upload(h.ksrcs);

@@ -34,6 +34,7 @@ struct DevPlan {
     float2* opmat32 = nullptr;     // FP32 copy of the operator table (mixed modes; MIXED: its uploaded part)
     float2* oppack = nullptr;      // packed operator blocks of the GEMMs: FP32 (MIXED translations)
     double2* oppack64 = nullptr;   // and FP64 (every other GEMM but the split-BF16 ones)
+    double2* zeros = nullptr;      // what the GEMMs read as absent blocks of B
     void* opmatbf = nullptr;       // split-BF16 copy (16 bytes per entry; mixed-split mode)
     KTask* ktasks = nullptr;
     KSrc* ksrcs = nullptr;

@@ -687,12 +687,19 @@ constexpr int MAXKB = 8;           // at most 8 K blocks (children of a box)
 // stall together at the barriers.  Translations alone, LDS form -> this one: 4M points x 8
 // RHS 28.9 -> 23.4 ms, 250k x 64 RHS 58.9 -> 43.7 ms, 1M x 1 RHS 5.9 -> 4.5 ms.
 //
-// Bounds of the loads: A is read without predicates; rows past the group's last one and k
-// past a segment's end read on into the table, whose end is padded with zeros (opmat_pad), or
-// a packed block's zeros; such rows are not stored, and such k meet zeros in B.  B is clamped
-// to the segment, and entries past it and those of absent columns (which read the buffer's
-// start) are replaced by zeros.  A column's order of k depends on G3M alone, so neither MB
-// nor CB changes a bit (the instruction itself sums its k in order by fma).
+// Launches of a wave or less per SIMD are bound by that wave's own instructions: beside 106
+// ns of FP64 (40 of FP32) MFMAs a k step of one row block took 80 (65) ns of address
+// arithmetic, clamps and selects, which only other waves can hide.  So little of that is left
+// in a step: absent blocks and columns point to a block of zeros, and the loads run up to a
+// step past a segment's end, at constant offsets from one pointer per column block.  FP64 U2U
+// of 6k points 0.105 -> 0.084 ms, of 60k 0.35 -> 0.30, 1M x 1 RHS 2.04 -> 1.95.
+//
+// Bounds of the loads: B up to GEMM_AHEAD k past the segment, in the slack behind each
+// buffer at its end (BUF_SLACK), and replaced by zeros from the segment's end on; A up to
+// the step's end, in the slack behind the packed tables (and, as stored, behind the
+// table, which is cleared first); row blocks past the group's last one are never read, rows past
+// it not stored.  A column's order of k depends on G3M alone, so neither MB nor CB changes a
+// bit (the instruction itself sums its k in order by fma).
 // Two adjacent FP32 complex values by one 16-byte load (global loads need dword alignment
 // only).
 struct CPair {
@@ -715,12 +722,14 @@ template <class TA, class V, class R, int MB, int CB, bool PACK, bool G3M>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(
     const GGroup* __restrict__ groups, const GTile* __restrict__ tiles,
     const int64_t* __restrict__ colB, const int64_t* __restrict__ colC, const int64_t* __restrict__ colA,
-    const TA* __restrict__ opm, const double2* __restrict__ scl, BufTable bt, int tile0, int nr) {
+    const TA* __restrict__ opm, const double2* __restrict__ scl, const void* __restrict__ zeros, BufTable bt,
+    int tile0, int nr) {
     using M = Mfma<R>;
     using T = typename Real<V>::T;
     constexpr int TN = GEMM_TN * CB;
     constexpr int UQ = sizeof(R) == 4 ? 2 : 1, UK = 4 * UQ;          // k steps and k per unit
     constexpr int NU = gemm_units(MB, CB), KQ = NU * UQ, KS = NU * UK;   // per pipeline step
+    static_assert(KS <= GEMM_AHEAD, "a step's loads stay in the slack");
     // k order of a unit: with three products lane group lk takes k = 2 lk + q in k step q (one
     // 16-byte load of B; a last unit of at most 4 k runs k = lk alone), with four k = lk + 4 q
     constexpr bool PAIR = G3M;
@@ -742,7 +751,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     const int64_t sB = bt.stride[g.bbuf], sC = bt.stride[g.cbuf];
     const int kb = g.kb ? g.kb : g.K;                   // segment length
     const int nkb = g.kb ? g.K / g.kb : 1;
-    // B offsets of the wave's columns per K block, -1 = absent: written and read by this wave
+    // B offsets of the wave's columns per K block, -1 = absent (no block there, or past the
+    // group's last column: read as zeros): written and read by this wave
     __shared__ int64_t bo[4][MAXKB][16 * CB];
 
     int64_t coff[CB];                                   // this lane's output columns
@@ -801,37 +811,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     struct Step {                  // operands of one pipeline step
         TA a[KQ][MB];
         V b[KQ][CB];
-        bool p[CB];                // the column is present in the segment
         int kl;                    // k left in the segment
-        bool fix;                  // some entry of b must be zeroed
     };
-    // loader: the current segment's A block and columns, and the k range of the step
-    const int ktop = (kb - 1) / UK * UK;       // first k of a segment's last unit
+    // loader: A and, at this lane's k, B of the step, and the k left in the segment
     const TA* Ap = nullptr;
     const V* Bp[CB];
-    bool pres[CB];
-    bool allp = true;
-    int k0 = 0, kl = 0;            // first k of the step and k left in the segment
+    int kl = 0;
     auto segment = [&]() {
         const int h = __builtin_ctz(act);
         act &= act - 1;
         Ap = opm + (g.kb ? colA[g.acol0 + h] : g.aoff) + (PACK ? ROWS / 16 * tl.m0 : tl.m0);
-        k0 = 0;
         kl = kb;
-        bool all = true;
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
             const int64_t v = bo[wave][h][16 * c + li];
-            pres[c] = v >= 0;
-            all &= v >= 0;
-            Bp[c] = B + (v >= 0 ? v : 0);
+            Bp[c] = (v >= 0 ? B + v : (const V*)zeros) + lk;
         }
-        allp = __all(all);
     };
     auto advance = [&]() {         // false: there is no further step (the loader stays)
         if (kl > KS) {
-            k0 += KS;
             kl -= KS;
+            Ap += NU * ustep;
+#pragma unroll
+            for (int c = 0; c < CB; ++c) Bp[c] += KS;
             return true;
         }
         if (!act) return false;
@@ -843,25 +845,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     auto fetch = [&](Step& s) {
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-            const int ku = NU == 1 ? k0 : min(k0 + u * UK, ktop);
             if constexpr (PAIR) {
-                // the pair's second entry is at most kb (BUF_SLACK)
-                const int k = min(ku + (kb - ku <= 4 ? lk : 2 * lk), kb - 1);
+                const int o = u * UK + (kl - u * UK <= 4 ? 0 : lk);
 #pragma unroll
                 for (int c = 0; c < CB; ++c) {
-                    const CPair b = load_pair(Bp[c] + k);
+                    const CPair b = load_pair(Bp[c] + o);
                     s.b[u * UQ][c] = b.e[0];
                     s.b[u * UQ + UQ - 1][c] = b.e[1];
                 }
             } else {
 #pragma unroll
-                for (int q = 0; q < UQ; ++q) {
-                    const int k = min(ku + 4 * q + lk, kb - 1);
+                for (int q = 0; q < UQ; ++q)
 #pragma unroll
-                    for (int c = 0; c < CB; ++c) s.b[u * UQ + q][c] = Bp[c][k];
-                }
+                    for (int c = 0; c < CB; ++c) s.b[u * UQ + q][c] = Bp[c][u * UK + 4 * q];
             }
-            const TA* ap = Ap + (unsigned)(ku / UK) * ustep + ao;
+            const TA* ap = Ap + u * ustep + ao;
 #pragma unroll
             for (int a = 0; a < MB; ++a) {
                 if constexpr (PACK && sizeof(R) == 4) {
@@ -873,22 +871,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
                 }
             }
         }
-#pragma unroll
-        for (int c = 0; c < CB; ++c) s.p[c] = pres[c];
         s.kl = kl;
-        s.fix = kl < KS || !allp;
     };
     // sweeps over the row blocks, so consecutive MFMAs never accumulate into the same
     // registers; one row fragment serves the wave's CB column blocks
     auto compute = [&](Step& s) {
-        if (s.fix) {
+        if (s.kl < KS) {           // zeros past the segment's end
 #pragma unroll
             for (int q = 0; q < KQ; ++q) {
                 const int kl = s.kl - q / UQ * UK;     // k left from the unit's first
                 const int kq = PAIR && kl > 4 ? 2 * lk + q % UQ : 4 * (q % UQ) + lk;
 #pragma unroll
                 for (int c = 0; c < CB; ++c)
-                    if (!s.p[c] || kq >= kl) s.b[q][c] = mk<V>(0, 0);
+                    if (kq >= kl) s.b[q][c] = mk<V>(0, 0);
             }
         }
 #pragma unroll
@@ -994,7 +989,7 @@ void launch_gemm_form(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d
 #define DDFMM_GEMM_MB(X)                                                                                            \
     case X:                                                                                                         \
         gemm_kernel<TA, V, R, X, CB, PACK, G3M><<<grid, 256, 0, st>>>(d.groups, d.tiles, d.colB, d.colC, d.colA,   \
-                                                                      opm, d.opmat, d.bt, s.begin, nrhs);          \
+                                                                      opm, d.opmat, d.zeros, d.bt, s.begin, nrhs); \
         break;
     switch (s.mb) {
         DDFMM_GEMM_MB(1) DDFMM_GEMM_MB(2) DDFMM_GEMM_MB(3) DDFMM_GEMM_MB(4) DDFMM_GEMM_MB(5)

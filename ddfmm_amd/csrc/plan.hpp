@@ -95,7 +95,8 @@ struct PackA {
     int64_t src, dst;           // first element in the operator table / in the packed table
     int M, K, lda, trans;       // the block as stored
 };
-constexpr int BUF_SLACK = 1;    // elements behind each work buffer: a pair read at a slot's last entry
+constexpr int GEMM_AHEAD = 32;  // k that the GEMM may read past a segment (at most a pipeline step)
+constexpr int BUF_SLACK = GEMM_AHEAD;   // elements behind each work buffer
 
 // LF FFT-diagonal M2L (wave3d_eval.cpp:602-661)
 struct FftSrc {

@@ -573,12 +573,13 @@ struct Builder {
                 if (g.transA >= 2) {
                     const bool f32 = g.transA == 2;
                     return aoff >= 0 && aoff % 64 == 0 && g.lda == (g.M + 15) / 16 &&
-                           aoff + pack_elems(f32, g.M, kcols) <= (f32 ? pl.pack32_total : pl.pack64_total);
+                           aoff + pack_elems(f32, g.M, kcols + GEMM_AHEAD) <=
+                               (f32 ? pl.pack32_total : pl.pack64_total);
                 }
                 const int64_t last = g.transA ? aoff + (int64_t)(g.M - 1) * g.lda + kcols
                                               : aoff + (int64_t)(kcols - 1) * g.lda + g.M;
-                // the kernel reads whole row blocks of 16 and units of 4 k
-                const int64_t mr = (g.M + 15) / 16 * 16, kr = (kcols + 3) / 4 * 4;
+                // the kernel reads whole row blocks of 16 and up to GEMM_AHEAD past the last k
+                const int64_t mr = (g.M + 15) / 16 * 16, kr = kcols + GEMM_AHEAD;
                 const int64_t read = g.transA ? aoff + (mr - 1) * g.lda + kr : aoff + (kr - 1) * g.lda + mr;
                 return aoff >= 0 && last <= pl.opmat_total && g.lda >= (g.transA ? kcols : g.M) &&
                        read <= pl.opmat_total + pl.opmat_pad;
@@ -588,7 +589,7 @@ struct Builder {
                 need(g.bcol0 + (int64_t)g.ncols <= (int64_t)pl.colB.size(), "gemm B columns");
                 for (int n = 0; n < g.ncols; ++n) {
                     const int64_t b = pl.colB[g.bcol0 + n];
-                    need(b >= 0 && b + g.K <= bsize(g.bbuf), "gemm B range");
+                    need(b >= 0 && b + g.K <= bsize(g.bbuf) && g.K + GEMM_AHEAD <= pl.zeros, "gemm B range");
                 }
             } else {
                 const int nkb = g.K / g.kb;
@@ -598,7 +599,7 @@ struct Builder {
                 need(g.bcol0 + (int64_t)g.ncols * nkb <= (int64_t)pl.colB.size(), "gemm B blocks");
                 for (int64_t e = 0; e < (int64_t)g.ncols * nkb; ++e) {
                     const int64_t b = pl.colB[g.bcol0 + e];
-                    need(b >= -1 && b + g.kb <= bsize(g.bbuf), "gemm B block range");
+                    need(b >= -1 && b + g.kb <= bsize(g.bbuf) && g.kb + GEMM_AHEAD <= pl.zeros, "gemm B block range");
                 }
             }
         }
@@ -1750,6 +1751,12 @@ void Builder::pack_operators() {
         }
         st.trans = f32 ? 2 : 3;
     }
+    int64_t slack[2] = {0, 0};
+    for (int f32 = 0; f32 < 2; ++f32)
+        for (const PackA& p : f32 ? pl.pack32 : pl.pack64)
+            slack[f32] = std::max(slack[f32], pack_elems(f32, p.M, p.K + GEMM_AHEAD) - pack_elems(f32, p.M, p.K));
+    pl.pack64_total += slack[0];
+    pl.pack32_total += slack[1];
 }
 
 void Builder::finish(bool want_dump) {
@@ -1757,7 +1764,9 @@ void Builder::finish(bool want_dump) {
     pack_operators();
     for (const GGroup& g : pl.groups)
         if (g.transA < 2)
-            pl.opmat_pad = std::max(pl.opmat_pad, 16 * (int64_t)g.lda + 16);
+            pl.opmat_pad = std::max(pl.opmat_pad, GEMM_AHEAD * (int64_t)g.lda + 16);
+    for (const GGroup& g : pl.groups)
+        pl.zeros = std::max<int64_t>(pl.zeros, (g.kb ? g.kb : g.K) + GEMM_AHEAD);
     // ---------------- per-stage algorithmic work (per RHS)
     for (auto& st : pl.stages) stage_work(pl, st);
 

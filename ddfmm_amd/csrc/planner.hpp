@@ -43,7 +43,8 @@ struct HostPlan {
     int64_t opmat_total = 0;               // uploaded + generated
     int64_t opmat_up = 0;                  // uploaded part alone
     std::vector<PackA> pack32, pack64;     // operator blocks packed at setup, per table
-    int64_t pack32_total = 0, pack64_total = 0;
+    int64_t pack32_total = 0, pack64_total = 0;   // with the slack behind them (GEMM_AHEAD)
+    int64_t zeros = 0;                     // length of the GEMMs' block of zeros
     int64_t opmat_pad = 0;                 // zeros behind the table: the setup GEMMs read whole row blocks and units
     std::vector<int> grid;                 // FFT grid index tables
     std::vector<double> genpts;            // kernel-generation point table (xyz rows)
