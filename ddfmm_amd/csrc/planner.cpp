@@ -379,7 +379,7 @@ struct Builder {
             for (int t = b; t < e; ++t)
                 if (lg.groups.empty() || lg.groups.back() != pl.tiles[t].g) lg.groups.push_back(pl.tiles[t].g);
             std::strncpy(lg.name, name, sizeof(lg.name) - 1);
-            resplit_rows(b, e);
+            set_heights(b, e, s.prec);
             s.end = (int)pl.tiles.size();
             lg.mbmax = 0;
             for (int t = b; t < s.end; ++t) lg.mbmax = std::max(lg.mbmax, pl.tiles[t].mb);
@@ -390,24 +390,81 @@ struct Builder {
         }
         pl.stages.push_back(s);
     }
-    // A GEMM stage whose launch (tiles x right-hand sides) has fewer than MIN_GEMM_TILES
-    // tiles (an LF level's M2M over a few hundred boxes) would leave most CUs idle: its
-    // groups' rows are split into proportionally more, shorter tiles (the tiles of the
-    // range are the last ones added).
+    // Tiles of a GEMM stage under the height limit that the estimate below finds fastest.  In k
+    // steps of one row block: the stage's work over the 1024 SIMDs, each height weighed by the
+    // time per row block that full launches take at it, plus the end of the launch, where its
+    // longest wave runs among others on its SIMD: twice that wave's length where all waves
+    // run the same K, five times where K is blocked (waves run the blocks present in their
+    // columns, and the long ones start late as often as early).  Tall tiles read B fewer
+    // times, short ones leave shorter ends; enough tiles for all CUs, the rule before, left
+    // U2U and L2L of small and middling trees at heights whose ends took as long as the rest.
+    // U2U alone, before -> after: 60k x 3 RHS 0.39 -> 0.33 ms, 147k x 1 0.61 -> 0.55, 1M x 1
+    // 1.95 -> 1.79, FP64 200k x 5 4.5 -> 4.0.  (An end per launched height instead, as the heights
+    // of a stage run one after the other: the stages alone take the same, whole passes
+    // 2-4% more, since the other stream's work fills the ends.)  The split-BF16 kernel, whose
+    // blocks share their tiles in LDS, keeps the rule before, at least MIN_GEMM_TILES tiles
+    // times right-hand sides (147k x 1: 3.20 ms, with this one 3.53).
     static constexpr int MIN_GEMM_TILES = 2048;
-    void resplit_rows(int b, int e) {
-        if ((int64_t)(e - b) * std::max(1, prm.nrhs_max) >= MIN_GEMM_TILES || e != (int)pl.tiles.size() || e <= b)
-            return;
+    void set_heights(int b, int e, int prec) {
+        static const double w32[GEMM_MB] = {1.85, 1.31, 1.14, 1.10, 1.09, 1.02, 1.00};
+        static const double w64[GEMM_MB] = {1.35, 1.15, 1.10, 1.08, 1.07, 1.04, 1.00};
+        if (e != (int)pl.tiles.size() || e <= b) return;
+        const double* wt = prec == PREC_TRANSLATION && prm.xlat > 0 ? w32 : w64;
+        const bool by_count = prec == PREC_TRANSLATION && prm.xlat == 2;
         std::vector<int> gs;
         for (int t = b; t < e; ++t)
             if (gs.empty() || gs.back() != pl.tiles[t].g) gs.push_back(pl.tiles[t].g);
-        const int64_t want = MIN_GEMM_TILES / std::max(1, prm.nrhs_max);
-        const int f = (int)((want + (e - b) - 1) / (e - b));
+        const int nr = std::max(1, prm.nrhs_max);
+        const int per = std::max(1, 16 / nr);            // boxes per wave
+        struct Chains { int mbt; double sum, longest; };  // k steps of a group's waves, per row block
+        std::vector<Chains> ch;
+        bool blocked = false;
+        for (int gi : gs) {
+            const GGroup& g = pl.groups[gi];
+            const int nkb = g.kb ? g.K / g.kb : 1, steps = ((g.kb ? g.kb : g.K) + 3) / 4;
+            Chains c{(g.M + 15) / 16, 0, 0};
+            blocked |= g.kb > 0;
+            for (int n0 = 0; n0 < g.ncols; n0 += GEMM_TN)
+                for (int n = n0, n1 = std::min(n0 + GEMM_TN, g.ncols); n < n1; n += per) {
+                    const int m = std::min(n + per, n1);
+                    int present = g.kb ? 0 : 1;
+                    for (int h = 0; g.kb && h < nkb; ++h) {
+                        bool any = false;
+                        for (int q = n; q < m && !any; ++q) any = pl.colB[g.bcol0 + (int64_t)q * nkb + h] >= 0;
+                        present += any;
+                    }
+                    c.sum += (double)present * steps * std::max(1.0, (double)(m - n) * nr / 16);
+                    c.longest = std::max(c.longest, (double)present * steps);
+                }
+            ch.push_back(c);
+        }
+        int best = GEMM_MB;
+        double tbest = 0;
+        for (int m = GEMM_MB; m >= 1; --m) {
+            double sum = 0, end = 0;
+            auto add = [&](const Chains& c, int height, int tiles) {
+                if (tiles == 0) return;
+                sum += c.sum * height * wt[height - 1] * tiles;
+                end = std::max(end, c.longest * height);
+            };
+            for (const Chains& c : ch) {
+                const int nmt = (c.mbt + m - 1) / m, lo = c.mbt / nmt, taller = c.mbt % nmt;
+                add(c, lo, nmt - taller);
+                add(c, lo + 1, taller);
+            }
+            const double t = sum / 1024 + (blocked ? 5 : 2) * end;
+            if (m == GEMM_MB || t < tbest) {
+                best = m;
+                tbest = t;
+            }
+        }
+        const int64_t launched = (int64_t)(e - b) * nr;
+        const int f = launched < MIN_GEMM_TILES ? (int)((MIN_GEMM_TILES / nr + (e - b) - 1) / (e - b)) : 1;
         pl.tiles.resize(b);
         for (int gi : gs) {
             const GGroup& g = pl.groups[gi];
             const int mbt = (g.M + 15) / 16;
-            const int nmt = std::min(mbt, (mbt + GEMM_MB - 1) / GEMM_MB * f);
+            const int nmt = by_count ? std::min(mbt, (mbt + GEMM_MB - 1) / GEMM_MB * f) : (mbt + best - 1) / best;
             const int nt = (g.ncols + GEMM_TN - 1) / GEMM_TN;
             for (int a = 0, b0 = 0; a < nmt; ++a) {
                 const int mb = (mbt - b0 + (nmt - a) - 1) / (nmt - a);
