@@ -738,13 +738,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     // becomes ceil(nr / CB) launched tiles of TN such columns; waves past its boxes or the
     // group's last column exit at once.
     const int per = (nr + CB - 1) / CB;
-    const int bx = xcd_chunk<GEMM_XCD_CHUNK / CB>(blockIdx.x, gridDim.x);
+    const bool one = blockDim.x == 64;                 // a block per wave (launch_gemm_form)
+    constexpr int CH = GEMM_XCD_CHUNK / CB;
+    const int it = one ? xcd_chunk<4 * CH>(blockIdx.x, gridDim.x) : 4 * xcd_chunk<CH>(blockIdx.x, gridDim.x);
+    const int bx = it >> 2;
     const GTile tl = tiles[tile0 + bx / per];
     const GGroup g = groups[tl.g];
     const int ncx = min(g.ncols, tl.n0 + GEMM_TN) * nr;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lk = lane >> 4;
-    const int n0 = tl.n0 * nr + TN * (bx % per) + 16 * CB * wave;    // the wave's first column
+    const int n0 = tl.n0 * nr + TN * (bx % per) + 16 * CB * (one ? it & 3 : wave);   // the wave's first column
     if (n0 >= ncx) return;
     const V* B = bufp<V>(bt, g.bbuf);
     V* C = bufp<V>(bt, g.cbuf);
@@ -983,13 +986,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     }
 }
 
+// From 16 right-hand sides up, where a wave's 16 columns are one box's and tiles fill whole
+// waves, each FP32 wave is a block of its own: the waves share nothing but cache lines, and a
+// block of four is not placed before a slot is free on every SIMD, nor its slots reused before
+// its last wave ends (e^{ikr} 250k x 16 RHS 29.6 -> 28.6 ms, 250k x 64 66.7 -> 66.4).  Below,
+// blocks of one gain nothing (4M x 8: the same) or lose: FP64 200k x 5 17.1 -> 17.7, as they leave
+// the other stream's large blocks no room, and with most tiles filling one wave of four
+// the waves with work fall on a quarter of the CUs (1M x 1 6.6 -> 7.4).
 template <class TA, class V, class R, int CB, bool PACK, bool G3M>
 void launch_gemm_form(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d, const TA* opm) {
-    const dim3 grid((s.end - s.begin) * ((nrhs + CB - 1) / CB), 1);
+    const bool one = sizeof(R) == 4 && nrhs >= 16;
+    const dim3 grid((s.end - s.begin) * ((nrhs + CB - 1) / CB) * (one ? 4 : 1), 1), block(one ? 64 : 256);
 #define DDFMM_GEMM_MB(X)                                                                                            \
     case X:                                                                                                         \
-        gemm_kernel<TA, V, R, X, CB, PACK, G3M><<<grid, 256, 0, st>>>(d.groups, d.tiles, d.colB, d.colC, d.colA,   \
-                                                                      opm, d.opmat, d.zeros, d.bt, s.begin, nrhs); \
+        gemm_kernel<TA, V, R, X, CB, PACK, G3M><<<grid, block, 0, st>>>(d.groups, d.tiles, d.colB, d.colC, d.colA,  \
+                                                                        opm, d.opmat, d.zeros, d.bt, s.begin, nrhs); \
         break;
     switch (s.mb) {
         DDFMM_GEMM_MB(1) DDFMM_GEMM_MB(2) DDFMM_GEMM_MB(3) DDFMM_GEMM_MB(4) DDFMM_GEMM_MB(5)
