@@ -115,6 +115,20 @@ struct ddfmm_ctx {
     }
 };
 
+// A device table that lives during setup only: freed when it leaves its scope, also when a
+// HIP call fails before its end.
+template <class T>
+struct SetupTable {
+    T* p = nullptr;
+    explicit SetupTable(int64_t n) { HIPCHK(hipMalloc(&p, (size_t)n * sizeof(T))); }
+    explicit SetupTable(const std::vector<T>& v) : SetupTable((int64_t)v.size()) {
+        HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+    }
+    ~SetupTable() { (void)hipFree(p); }
+    SetupTable(const SetupTable&) = delete;
+    SetupTable& operator=(const SetupTable&) = delete;
+};
+
 // Device bytes of a set-up context: `fixed` for the point, operator and descriptor
 // tables (kept for the context's life), `per_rhs` for the work buffers and the staging
 // of one right-hand side, `transient` for the generator tables that live only during
@@ -337,16 +351,10 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         d.io = c->alloc<IoPtrs>(1);
         // translation matrices generated on the device (temporary generator tables)
         if (!h.kgen.empty()) {
-            double* gp = nullptr;
-            KGen* jobs = nullptr;
-            HIPCHK(hipMalloc(&gp, h.genpts.size() * sizeof(double)));
-            HIPCHK(hipMalloc(&jobs, h.kgen.size() * sizeof(KGen)));
-            HIPCHK(hipMemcpy(gp, h.genpts.data(), h.genpts.size() * sizeof(double), hipMemcpyHostToDevice));
-            HIPCHK(hipMemcpy(jobs, h.kgen.data(), h.kgen.size() * sizeof(KGen), hipMemcpyHostToDevice));
-            HIPCHK(launch_kgen(jobs, (int)h.kgen.size(), gp, d.opmat, d.ktype, c->stream));
+            const SetupTable<double> gp(h.genpts);
+            const SetupTable<KGen> jobs(h.kgen);
+            HIPCHK(launch_kgen(jobs.p, (int)h.kgen.size(), gp.p, d.opmat, d.ktype, c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
-            HIPCHK(hipFree(gp));
-            HIPCHK(hipFree(jobs));
         }
         // fused mode: solves folded into the translations by FP64 GEMMs on the table
         if (!h.setup_stages.empty()) {
@@ -371,13 +379,10 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         for (int f32 = 0; f32 < 2; ++f32) {
             const std::vector<PackA>& pk = f32 ? h.pack32 : h.pack64;
             if (pk.empty()) continue;
-            PackA* jobs = nullptr;
-            HIPCHK(hipMalloc(&jobs, pk.size() * sizeof(PackA)));
-            HIPCHK(hipMemcpy(jobs, pk.data(), pk.size() * sizeof(PackA), hipMemcpyHostToDevice));
-            HIPCHK(launch_pack(jobs, (int)pk.size(), d.opmat, f32 ? (void*)d.oppack : (void*)d.oppack64, f32,
+            const SetupTable<PackA> jobs(pk);
+            HIPCHK(launch_pack(jobs.p, (int)pk.size(), d.opmat, f32 ? (void*)d.oppack : (void*)d.oppack64, f32,
                                d.ktype == 0, c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
-            HIPCHK(hipFree(jobs));
         }
         // work buffers, after the setup-time tables are gone
         for (int b = 0; b < BUF_COUNT; ++b) {

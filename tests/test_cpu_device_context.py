@@ -1,0 +1,80 @@
+"""What a device context allocates, frees and waits for, without a GPU: the library runs on
+a stand-in for the HIP runtime (cxx/host_hip.cpp, host memory, kernels that do nothing), in
+a process of its own that loads the stand-in first."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+
+PRELUDE = """
+import ctypes, sys
+hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+for f in ("live", "peak", "calls", "early"):
+    getattr(hip, "host_hip_" + f).restype = ctypes.c_int64
+for f in ("fail", "free_bytes"):
+    getattr(hip, "host_hip_" + f).argtypes = [ctypes.c_int64]
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from ddfmm_amd import geometry
+from ddfmm_amd._lib import DdfmmError, lib
+from ddfmm_amd.wave3d import FP64, FP64_FUSED, MIXED, MIXED_SPLIT, Mlib3d, Wave3d
+
+K, N = 2.0, 1500
+ml = Mlib3d()
+ml.setup({"-mlib3d_ldname": sys.argv[3], "-mlib3d_hdname": sys.argv[4]})
+
+def wave(precision, nrhs=1, budget=0, device=0, k=K, n=N):
+    w = Wave3d(device=device)
+    w.posptr, w.mlibptr = geometry.sphere(n, k, 81), ml
+    w.setup({"-wave3d_ACCU": 2, "-wave3d_K": k, "-wave3d_maxlevel": 12, "-wave3d_hbm_budget": budget / 2**30},
+            nrhs_max=nrhs, precision=precision)
+    return w
+"""
+
+
+@pytest.fixture(scope="module")
+def host_hip(tmp_path_factory):
+    so = tmp_path_factory.mktemp("hip") / "libamdhip64.so.7"
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", os.path.join(HERE, "cxx", "host_hip.cpp"), "-o", str(so),
+                    "-Wl,-soname,libamdhip64.so.7",
+                    "-Wl,--version-script=" + os.path.join(HERE, "cxx", "host_hip.map")], check=True)
+    return str(so)
+
+
+@pytest.fixture
+def run(host_hip, oplib):
+    def go(code):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + code, host_hip, ROOT, oplib[0], oplib[1]],
+                           capture_output=True, text=True, timeout=300)
+        print(r.stdout, flush=True)
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+        return r.stdout
+    return go
+
+
+def test_failed_setup_frees_everything(run):
+    """Each HIP call of a setup fails in turn: setup reports the error and no allocation is
+    left (its temporary tables among them), nor after the contexts that work."""
+    run("""
+for p in (FP64, MIXED, FP64_FUSED, MIXED_SPLIT):
+    hip.host_hip_reset()
+    w = wave(p)
+    n = hip.host_hip_calls()
+    w.close()
+    assert hip.host_hip_live() == 0, (p, hip.host_hip_live())
+    for i in range(1, n + 1):
+        hip.host_hip_fail(i)
+        try:
+            wave(p)
+            assert False, ("no error", p, i)
+        except DdfmmError as e:
+            assert "out of memory" in str(e), (p, i, str(e))
+        assert hip.host_hip_live() == 0, (p, i, n, hip.host_hip_live())
+    print("precision", p, "calls", n, flush=True)
+""")
