@@ -541,8 +541,9 @@ struct Builder {
     void finish(bool want_dump);
 
     // Every descriptor's element range must lie inside the buffer or table it indexes: the
-    // kernels trust these offsets, so a planner mistake is caught here on the host.
-    void validate() const {
+    // kernels trust these offsets, so a planner mistake is caught here on the host.  Row scales
+    // and V-list tables lie in the table's uploaded part, the only one copied in FP32.
+    static void validate(const HostPlan& pl) {
         auto need = [](bool ok, const char* what) {
             if (!ok) throw Error(std::string("internal: descriptor out of bounds (") + what + ")");
         };
@@ -625,7 +626,7 @@ struct Builder {
                 const int64_t c = pl.colC[g.col0 + n];
                 need(c >= 0 && c + g.M <= bsize(g.cbuf), "gemm C range");
             }
-            if (g.soff >= 0) need(g.soff + g.M <= pl.opmat_total, "gemm row scale");
+            if (g.soff >= 0) need(g.soff + g.M <= pl.opmat_up, "gemm row scale");
             auto a_ok = [&](int64_t aoff, int kcols) {
                 if (g.transA >= 2) {
                     const bool f32 = g.transA == 2;
@@ -687,7 +688,7 @@ struct Builder {
         }
         for (const VTarget& v : pl.vtrg) {
             need(v.out_off >= 0 && v.out_off + pl.NL <= pl.bufsize[BUF_LF_CHK], "vlist out");
-            need(v.tab_off >= 0 && v.tab_off + 343 * G3 <= pl.opmat_total, "vlist table");
+            need(v.tab_off >= 0 && v.tab_off + 343 * G3 <= pl.opmat_up, "vlist table");
             need(v.grid >= 0 && v.grid + pl.NL <= (int64_t)pl.grid.size(), "vlist grid");
             need(v.p0 >= 0 && v.p0 <= v.p1 && v.p1 <= (int)pl.vpair.size(), "vlist pairs");
             for (int q = v.p0; q < v.p1; ++q) {
@@ -1827,7 +1828,7 @@ void Builder::finish(bool want_dump) {
     // ---------------- per-stage algorithmic work (per RHS)
     for (auto& st : pl.stages) stage_work(pl, st);
 
-    validate();
+    validate(pl);
 
     // ---------------- canonical dump of the lists (integer parity with the oracle)
     if (want_dump) {
@@ -1868,5 +1869,7 @@ void build_plan(const Params& prm, const double* pos, int64_t N, const Mlib& mli
     Builder b(prm, mlib, plan);
     b.run(pos, N, want_dump);
 }
+
+void validate_plan(const HostPlan& plan) { Builder::validate(plan); }
 
 }  // namespace ddfmm

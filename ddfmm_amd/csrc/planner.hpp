@@ -73,6 +73,10 @@ struct HostPlan {
 void build_plan(const Params& prm, const double* pos, int64_t N, const Mlib& mlib,
                 HostPlan& plan, bool want_dump);
 
+// Throws unless every descriptor's range lies inside the buffer or table it indexes
+// (build_plan ends with it).
+void validate_plan(const HostPlan& plan);
+
 // Algorithmic work per RHS of a stage (Stage::work) and, for GEMM stages, the MFMA flops
 // the kernel executes under its tiling (Stage::exec).
 void stage_work(const HostPlan& plan, Stage& s);
