@@ -120,9 +120,11 @@ struct ddfmm_ctx {
 template <class T>
 struct SetupTable {
     T* p = nullptr;
-    explicit SetupTable(int64_t n) { HIPCHK(hipMalloc(&p, (size_t)n * sizeof(T))); }
+    explicit SetupTable(int64_t n) {
+        if (n > 0) HIPCHK(hipMalloc(&p, (size_t)n * sizeof(T)));
+    }
     explicit SetupTable(const std::vector<T>& v) : SetupTable((int64_t)v.size()) {
-        HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+        if (p) HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
     }
     ~SetupTable() { (void)hipFree(p); }
     SetupTable(const SetupTable&) = delete;
@@ -131,25 +133,23 @@ struct SetupTable {
 
 // Device bytes of a set-up context: `fixed` for the point, operator and descriptor
 // tables (kept for the context's life), `per_rhs` for the work buffers and the staging
-// of one right-hand side, `transient` for the generator tables that live only during
-// setup (freed before the work buffers are allocated).
+// of one right-hand side, `transient` for what lives only during setup (freed before the
+// work buffers are allocated): the window of the operator table's generated part that is
+// being made, the generator tables and the packing jobs.
 template <class T>
 static int64_t vbytes(const std::vector<T>& v) { return (int64_t)v.size() * (int64_t)sizeof(T); }
 static void plan_bytes(const HostPlan& h, int precision, int64_t& fixed, int64_t& per_rhs, int64_t& transient) {
     const bool mixed = precision == DDFMM_MIXED || precision == DDFMM_MIXED_SPLIT;
     fixed = vbytes(h.px) + vbytes(h.py) + vbytes(h.pz) + 2 * vbytes(h.perm) + vbytes(h.grid) +
-            (h.opmat_total + h.opmat_pad) * (int64_t)sizeof(double2) +
-            (mixed ? (h.prm.xlat == 1 ? h.opmat_up : h.opmat_total) * (int64_t)sizeof(float2) : 0) +
-            h.pack32_total * (int64_t)sizeof(float2) + (h.pack64_total + h.zeros) * (int64_t)sizeof(double2) +
+            (h.opmat_up + h.zeros) * (int64_t)sizeof(double2) + (mixed ? h.opmat_up * (int64_t)sizeof(float2) : 0) +
+            h.pack32_total * (int64_t)sizeof(float2) + h.pack64_total * (int64_t)sizeof(double2) +
             (precision == DDFMM_MIXED_SPLIT ? h.opmat_total * 16 : 0) +
             vbytes(h.ktasks) + vbytes(h.ksrcs) + vbytes(h.groups) + vbytes(h.tiles) + vbytes(h.colB) +
             vbytes(h.colC) + vbytes(h.colA) + vbytes(h.fsrc) + vbytes(h.vtrg) + vbytes(h.vchunk) +
             vbytes(h.vsrc) + vbytes(h.vpk) + vbytes(h.rtrg) + (int64_t)sizeof(IoPtrs);
-    const int64_t esz = mixed ? (int64_t)sizeof(float2) : (int64_t)sizeof(double2);
-    per_rhs = 2 * h.N * (int64_t)sizeof(double2);
-    for (int b = 0; b < BUF_COUNT; ++b) per_rhs += h.bufsize[b] * esz;
-    for (int b = 0; b < BUF_COUNT; ++b) fixed += h.bufsize[b] > 0 ? BUF_SLACK * esz : 0;
-    transient = std::max(vbytes(h.genpts) + vbytes(h.kgen), std::max(vbytes(h.pack32), vbytes(h.pack64)));
+    per_rhs = h.rhs_bytes();
+    for (int b = 0; b < BUF_COUNT; ++b) fixed += h.bufsize[b] > 0 ? BUF_SLACK * h.vector_bytes() : 0;
+    transient = h.setup_bytes() + (h.windows.empty() ? 0 : (h.window_elems + GEMM_AHEAD) * (int64_t)sizeof(double2));
 }
 
 // The kernel-apply flavour is fixed per context (each right-hand side then has the same
@@ -287,6 +287,7 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         // leaves of up to 128 points most pairs qualify (with larger leaves few do, and the
         // reduction of the mirror products costs more than it saves)
         q.near_pairs = kapply_on_mfma(p->precision, p->nrhs_max) && p->ptsmax <= 2 * MIRROR_MAX_TARGETS;
+        q.budget = c->hbm_budget > 0;
         c->nrhs_max = p->nrhs_max;
         c->precision = p->precision;
         std::shared_ptr<const Mlib> mlib = shared ? shared : load_mlib(ldfile, hdfile);
@@ -332,13 +333,13 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
             d.iperm = c->upload(iperm);
         }
         d.grid = c->upload(h.grid);
-        const int64_t table = h.opmat_total + h.opmat_pad;
-        d.opmat = c->alloc<double2>(table);
-        // cleared: the setup's products read up to a row block and k step past a block, where
-        // the table may not be written yet, and multiply such k with zeros
-        HIPCHK(hipMemset(d.opmat, 0, (size_t)table * sizeof(double2)));
-        d.zeros = c->alloc<double2>(h.zeros);
-        HIPCHK(hipMemset(d.zeros, 0, (size_t)h.zeros * sizeof(double2)));
+        // the window's memory first and, without a budget, given back last: taken after the
+        // large tables, or freed before the work buffers, it cost 2 ms of a setup of 13
+        auto window = std::make_unique<SetupTable<double2>>(h.windows.empty() ? 0 : h.window_elems + GEMM_AHEAD);
+        // uploaded part of the operator table, the GEMMs' zeros behind it
+        d.opmat = c->alloc<double2>(h.opmat_up + h.zeros);
+        d.zeros = d.opmat + h.opmat_up;
+        if (h.zeros > 0) HIPCHK(hipMemset(d.zeros, 0, (size_t)h.zeros * sizeof(double2)));
         if (!h.opmat.empty())
             HIPCHK(hipMemcpy(d.opmat, h.opmat.data(), h.opmat.size() * sizeof(double2), hipMemcpyHostToDevice));
         d.ktasks = c->upload(h.ktasks); d.ksrcs = c->upload(h.ksrcs);
@@ -349,41 +350,44 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         d.vchunk = c->upload(h.vchunk); d.vsrc = c->upload(h.vsrc); d.vpk = c->upload(h.vpk);
         d.rtrg = c->upload(h.rtrg);
         d.io = c->alloc<IoPtrs>(1);
-        // translation matrices generated on the device (temporary generator tables)
-        if (!h.kgen.empty()) {
-            const SetupTable<double> gp(h.genpts);
-            const SetupTable<KGen> jobs(h.kgen);
-            HIPCHK(launch_kgen(jobs.p, (int)h.kgen.size(), gp.p, d.opmat, d.ktype, c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
-        }
-        // fused mode: solves folded into the translations by FP64 GEMMs on the table
-        if (!h.setup_stages.empty()) {
-            d.bt.p[BUF_OPMAT] = d.opmat;
-            d.bt.stride[BUF_OPMAT] = 0;
-            for (const Stage& s : h.setup_stages) HIPCHK(launch_setup_gemm(d, s, c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
-        }
         if (d.mixed) {
-            const int64_t n32 = h.prm.xlat == 1 ? h.opmat_up : h.opmat_total;
-            d.opmat32 = c->alloc<float2>(n32);
-            HIPCHK(launch_to_f32(d.opmat, d.opmat32, n32, c->stream));
+            d.opmat32 = c->alloc<float2>(h.opmat_up);
+            HIPCHK(launch_to_f32(d.opmat, d.opmat32, h.opmat_up, c->stream));
             if (c->precision == DDFMM_MIXED_SPLIT) {    // translations as split-BF16 products
                 d.opmatbf = (void*)c->alloc<double2>(h.opmat_total);
-                HIPCHK(launch_to_bf16s(d.opmat, d.opmatbf, h.opmat_total, c->stream));
+                HIPCHK(launch_to_bf16s(d.opmat, d.opmatbf, h.opmat_up, c->stream));
             }
-            HIPCHK(hipStreamSynchronize(c->stream));
         }
         // the GEMMs' operators in lane order (three products, e^{ikr}/r in FP32, take k in pairs)
         d.oppack = c->alloc<float2>(h.pack32_total);
         d.oppack64 = c->alloc<double2>(h.pack64_total);
-        for (int f32 = 0; f32 < 2; ++f32) {
-            const std::vector<PackA>& pk = f32 ? h.pack32 : h.pack64;
-            if (pk.empty()) continue;
-            const SetupTable<PackA> jobs(pk);
-            HIPCHK(launch_pack(jobs.p, (int)pk.size(), d.opmat, f32 ? (void*)d.oppack : (void*)d.oppack64, f32,
-                               d.ktype == 0, c->stream));
+        {
+            const SetupTable<double> gp(h.genpts);
+            const SetupTable<KGen> kgen(h.kgen);
+            const SetupTable<PackA> jobs64(h.pack64), jobs32(h.pack32);
+            auto pack = [&](const double2* from, const int* p0, const int* p1) {
+                HIPCHK(launch_pack(jobs64.p + p0[0], p1[0] - p0[0], from, d.oppack64, 0, 0, c->stream));
+                HIPCHK(launch_pack(jobs32.p + p0[1], p1[1] - p0[1], from, d.oppack, 1, d.ktype == 0, c->stream));
+            };
+            const int none[2] = {0, 0};
+            pack(d.opmat, none, h.pack_up);
+            // the generated part, one window after the other in the same memory: kernel
+            // matrices, fused operators (solves folded into the translations by FP64 GEMMs),
+            // packed blocks
+            d.bt.p[BUF_OPMAT] = d.opmat;
+            for (const SetupWindow& w : h.windows) {
+                double2* gen = window->p - w.begin;     // indexed by table offsets of the window
+                d.bt.p[BUF_OPGEN] = gen;
+                HIPCHK(launch_kgen(kgen.p + w.k0, w.k1 - w.k0, gp.p, gen, d.ktype, c->stream));
+                for (int q = w.s0; q < w.s1; ++q) HIPCHK(launch_setup_gemm(d, h.setup_stages[q], c->stream));
+                pack(gen, w.p0, w.p1);
+                if (d.opmatbf)
+                    HIPCHK(launch_to_bf16s(window->p, (double2*)d.opmatbf + w.begin, w.end - w.begin, c->stream));
+            }
+            d.bt.p[BUF_OPMAT] = d.bt.p[BUF_OPGEN] = nullptr;
             HIPCHK(hipStreamSynchronize(c->stream));
         }
+        if (c->hbm_budget > 0) window.reset();
         // work buffers, after the setup-time tables are gone
         for (int b = 0; b < BUF_COUNT; ++b) {
             d.bt.stride[b] = h.bufsize[b];

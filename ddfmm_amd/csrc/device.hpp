@@ -8,9 +8,9 @@
 namespace ddfmm {
 
 struct BufTable {
-    void* p[BUF_COUNT + 1];        // double2 (FP64 mode) or float2 (mixed mode) elements;
-                                   // p[BUF_OPMAT]: the FP64 operator table (setup GEMMs)
-    int64_t stride[BUF_COUNT + 1]; // elements per rhs slab
+    void* p[BUF_ALL];              // double2 (FP64 mode) or float2 (mixed mode) elements;
+                                   // BUF_OPMAT, BUF_OPGEN: the FP64 operator table (setup GEMMs)
+    int64_t stride[BUF_ALL];       // elements per rhs slab
 };
 
 // The caller's density and potential buffers of the current evaluation, read by the
@@ -30,12 +30,12 @@ struct DevPlan {
     int* perm = nullptr;           // sorted position -> input index
     int* iperm = nullptr;          // input index -> sorted position
     int* grid = nullptr;
-    double2* opmat = nullptr;
-    float2* opmat32 = nullptr;     // FP32 copy of the operator table (mixed modes; MIXED: its uploaded part)
+    double2* opmat = nullptr;      // uploaded part of the operator table
+    float2* opmat32 = nullptr;     // FP32 copy of it (mixed modes)
     float2* oppack = nullptr;      // packed operator blocks of the GEMMs: FP32 (MIXED translations)
     double2* oppack64 = nullptr;   // and FP64 (every other GEMM but the split-BF16 ones)
     double2* zeros = nullptr;      // what the GEMMs read as absent blocks of B
-    void* opmatbf = nullptr;       // split-BF16 copy (16 bytes per entry; mixed-split mode)
+    void* opmatbf = nullptr;       // split-BF16 copy of the whole table (16 bytes per entry; mixed-split mode)
     KTask* ktasks = nullptr;
     KSrc* ksrcs = nullptr;
     GGroup* groups = nullptr;
@@ -56,7 +56,8 @@ struct DevPlan {
 hipError_t launch_stage(const DevPlan& d, const Stage& s, int nrhs, hipStream_t st);
 hipError_t launch_set_io(IoPtrs* io, const double2* den, double2* val, hipStream_t st);
 hipError_t launch_setup_gemm(const DevPlan& d, const Stage& s, hipStream_t st);   // FP64, on the operator table
-hipError_t launch_kgen(const KGen* jobs, int njobs, const double* gp, double2* opmat, int ktype, hipStream_t st);
+// gen: the generated part's base, so that table offsets of the window in memory index it
+hipError_t launch_kgen(const KGen* jobs, int njobs, const double* gp, double2* gen, int ktype, hipStream_t st);
 // Direct sum split over S source ranges (chunk sources each, RC right-hand sides per
 // block); with S > 1 the ranges write part (S x nrhs x M complex, part_elems) and a
 // fixed-order reduction adds them into out.  The split depends on (M, Ns, nrhs) only, so

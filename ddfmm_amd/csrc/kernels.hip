@@ -695,10 +695,11 @@ constexpr int MAXKB = 8;           // at most 8 K blocks (children of a box)
 // of 6k points 0.105 -> 0.084 ms, of 60k 0.35 -> 0.30, 1M x 1 RHS 2.04 -> 1.95.
 //
 // Bounds of the loads: B up to GEMM_AHEAD k past the segment, in the slack behind each
-// buffer at its end (BUF_SLACK), and replaced by zeros from the segment's end on; A up to
-// the step's end, in the slack behind the packed tables (and, as stored, behind the
-// table, which is cleared first); row blocks past the group's last one are never read, rows past
-// it not stored.  A column's order of k depends on G3M alone, so neither MB nor CB changes a
+// buffer at its end (BUF_SLACK; the zeros behind the operator table, the setup window's
+// slack), and replaced by zeros from the segment's end on; packed A up to the step's end, in
+// the slack behind the packed tables, A as stored inside its block (what a zero of B
+// multiplies is the block's own); row blocks past the group's last one are never read, rows
+// past it not stored.  A column's order of k depends on G3M alone, so neither MB nor CB changes a
 // bit (the instruction itself sums its k in order by fma).
 // Two adjacent FP32 complex values by one 16-byte load (global loads need dword alignment
 // only).
@@ -716,8 +717,8 @@ __device__ __forceinline__ CPair load_pair(const float2* p) {
 // ms, of 60k 0.39 -> 0.35; twice as many units at one and two row blocks: 0.103 and 0.37.
 constexpr int gemm_units(int mb, int cb) { return cb > 1 || mb > 3 ? 1 : mb > 1 ? 2 : 4; }
 
-// PACK: A packed (PackA in plan.hpp) in the order the lanes take it; else as stored, column
-// major (the setup's products on the operator table itself).
+// PACK: A packed (PackA in plan.hpp) in the order the lanes take it; else as stored in the
+// operator table (the setup's products).
 template <class TA, class V, class R, int MB, int CB, bool PACK, bool G3M>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(
     const GGroup* __restrict__ groups, const GTile* __restrict__ tiles,
@@ -787,10 +788,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         }
         wave_lds_order();
     }
-    // A elements of this lane within a unit, per row block and per unit
-    constexpr unsigned ROWS = PACK ? 64 * UQ : 16;
+    // A elements of this lane within a unit, per row block and per unit.  As stored, rows
+    // past the group's last repeat that one, and k past the segment's end its first.
+    static_assert(PACK || sizeof(R) == 8, "operators as stored in FP64 only");
+    constexpr unsigned ROWS = 64 * UQ;
     const unsigned lda = g.lda;
-    const unsigned ao = PACK ? UQ * lane : lk * lda + li, ustep = PACK ? ROWS * lda : UK * lda;
+    const unsigned ustep = PACK ? ROWS * lda : UK * lda;
+    unsigned ao[PACK ? 1 : MB];
+    if constexpr (PACK) {
+        ao[0] = UQ * lane;
+    } else {
+#pragma unroll
+        for (int a = 0; a < MB; ++a) ao[a] = min(tl.m0 + 16 * a + li, g.M - 1);
+    }
 
     // G3M (FP32 contexts of the e^{ikr}/r kernel): three real products per complex one,
     // summed over k apart: k1 = (Ar + Ai) Br, k2 = Ar (Bi - Br), k3 = Ai (Br + Bi); Re C =
@@ -823,7 +833,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     auto segment = [&]() {
         const int h = __builtin_ctz(act);
         act &= act - 1;
-        Ap = opm + (g.kb ? colA[g.acol0 + h] : g.aoff) + (PACK ? ROWS / 16 * tl.m0 : tl.m0);
+        Ap = opm + (g.kb ? colA[g.acol0 + h] : g.aoff) + (PACK ? ROWS / 16 * tl.m0 : 0);
         kl = kb;
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
@@ -862,7 +872,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
                     for (int c = 0; c < CB; ++c) s.b[u * UQ + q][c] = Bp[c][u * UK + 4 * q];
             }
-            const TA* ap = Ap + u * ustep + ao;
+            const int left = kl - u * UK;          // k left from the unit's first
+            const TA* ap = PACK ? Ap + u * ustep + ao[0]
+                                : Ap + ((left > 0 ? u * ustep : 0) + (lk < left ? lk * lda : 0));
 #pragma unroll
             for (int a = 0; a < MB; ++a) {
                 if constexpr (PACK && sizeof(R) == 4) {
@@ -870,7 +882,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
                     s.a[u * UQ][a] = make_float2(v.x, v.y);
                     s.a[u * UQ + UQ - 1][a] = make_float2(v.z, v.w);
                 } else {
-                    s.a[u * UQ][a] = ap[ROWS * a];
+                    s.a[u * UQ][a] = ap[PACK ? ROWS * a : ao[PACK ? 0 : a]];
                 }
             }
         }
@@ -1022,6 +1034,11 @@ void launch_gemm32(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
         launch_gemm_form<float2, float2, float, 1, true, G3M>(s, nrhs, st, d, d.oppack);
 }
 
+// Blocks per kernel matrix or packed operator block at setup: a setup window holds a few
+// hundred of them, and one block each takes 20-90 dependent rounds for every window (6k points
+// in FP64, 7 windows: 0.3 ms for generation and packing, 0.65 with one block).
+constexpr int SETUP_SPLIT = 8;
+
 // One packed operator block per job (PackA): zeros past the block's edges.
 template <class T>
 __global__ __launch_bounds__(256) void pack_kernel(const PackA* __restrict__ jobs, const double2* __restrict__ opmat,
@@ -1029,7 +1046,7 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackA* __restrict__ job
     constexpr int UQ = 16 / (int)sizeof(T), UK = 4 * UQ;
     const PackA p = jobs[blockIdx.x];
     const int nrb = (p.M + 15) / 16, nk = (p.K + UK - 1) / UK;
-    for (int e = threadIdx.x; e < nrb * nk * 64 * UQ; e += 256) {
+    for (int e = blockIdx.y * 256 + threadIdx.x; e < nrb * nk * 64 * UQ; e += SETUP_SPLIT * 256) {
         const int q = e % UQ, lane = e / UQ & 63, rb = e / (64 * UQ) % nrb, o = e / (64 * UQ) / nrb;
         const int m = 16 * rb + (lane & 15), lk = lane >> 4;
         const int k = UK * o + (pair && p.K - UK * o > 4 ? 2 * lk + q : lk + 4 * q);
@@ -1731,17 +1748,17 @@ __global__ __launch_bounds__(256) void vlist_inv_kernel(const VTarget* __restric
 
 // ---------------------------------------------------------------- setup-time generation
 __global__ __launch_bounds__(256) void kgen_kernel(const KGen* __restrict__ jobs, const double* __restrict__ gp,
-                                                   double2* __restrict__ opmat, int j0, int ktype) {
+                                                   double2* __restrict__ gen, int j0, int ktype) {
     const KGen k = jobs[j0 + blockIdx.x];
     const double sg = k.tneg ? -1.0 : 1.0;
     const int64_t mn = (int64_t)k.m * k.n;
-    for (int64_t e = threadIdx.x; e < mn; e += blockDim.x) {
+    for (int64_t e = blockIdx.y * 256 + threadIdx.x; e < mn; e += SETUP_SPLIT * 256) {
         const int i = (int)(e % k.m), j = (int)(e / k.m);
         const double* t = gp + 3 * (k.toff + i);
         const double* s = gp + 3 * (k.soff + j);
         double d[3];
         for (int q = 0; q < 3; ++q) d[q] = (sg * t[q] + k.tshift[q]) - (s[q] + k.sshift[q]);
-        opmat[k.out + e] = green64_table(d[0], d[1], d[2], ktype);
+        gen[k.out + e] = green64_table(d[0], d[1], d[2], ktype);
     }
 }
 
@@ -2058,15 +2075,16 @@ hipError_t launch_stage(const DevPlan& d, const Stage& s, int nrhs, hipStream_t 
 }
 
 hipError_t launch_setup_gemm(const DevPlan& d, const Stage& s, hipStream_t st) {
-    if (s.kind != ST_GEMM || s.mb < 1 || s.mb > GEMM_MB) return hipErrorInvalidValue;
-    launch_gemm_form<double2, double2, double, 1, false, false>(s, 1, st, d, d.opmat);
+    if (s.kind != ST_GEMM || s.mb < 1 || s.mb > GEMM_MB || s.buf < BUF_OPMAT || s.buf >= BUF_ALL)
+        return hipErrorInvalidValue;
+    launch_gemm_form<double2, double2, double, 1, false, false>(s, 1, st, d, (const double2*)d.bt.p[s.buf]);
     return hipGetLastError();
 }
 
-hipError_t launch_kgen(const KGen* jobs, int njobs, const double* gp, double2* opmat, int ktype, hipStream_t st) {
+hipError_t launch_kgen(const KGen* jobs, int njobs, const double* gp, double2* gen, int ktype, hipStream_t st) {
     for (int j0 = 0; j0 < njobs; j0 += 65536) {
         int n = std::min(65536, njobs - j0);
-        kgen_kernel<<<n, 256, 0, st>>>(jobs, gp, opmat, j0, ktype);
+        kgen_kernel<<<dim3(n, SETUP_SPLIT), 256, 0, st>>>(jobs, gp, gen, j0, ktype);
     }
     return hipGetLastError();
 }
@@ -2074,8 +2092,9 @@ hipError_t launch_kgen(const KGen* jobs, int njobs, const double* gp, double2* o
 hipError_t launch_pack(const PackA* jobs, int njobs, const double2* opmat, void* out, int f32, int pair, hipStream_t st) {
     for (int j0 = 0; j0 < njobs; j0 += 65536) {
         const int n = std::min(65536, njobs - j0);
-        if (f32) pack_kernel<float2><<<n, 256, 0, st>>>(jobs + j0, opmat, (float2*)out, pair);
-        else pack_kernel<double2><<<n, 256, 0, st>>>(jobs + j0, opmat, (double2*)out, 0);
+        const dim3 grid(n, SETUP_SPLIT);
+        if (f32) pack_kernel<float2><<<grid, 256, 0, st>>>(jobs + j0, opmat, (float2*)out, pair);
+        else pack_kernel<double2><<<grid, 256, 0, st>>>(jobs + j0, opmat, (double2*)out, 0);
     }
     return hipGetLastError();
 }

@@ -28,8 +28,11 @@ enum Buf : int {
                     // slots into one leaf adjacent, in source-task order)
     BUF_COUNT
 };
-// setup-time GEMMs read and write the operator table itself (FP64), as buffer BUF_OPMAT
+// setup-time GEMMs read and write the operator table itself (FP64), as two buffers: its
+// uploaded part, and its generated part (offsets in the table; the window of it in memory)
 constexpr int BUF_OPMAT = BUF_COUNT;
+constexpr int BUF_OPGEN = BUF_COUNT + 1;
+constexpr int BUF_ALL = BUF_COUNT + 2;
 
 // near-field pairs evaluated once for both directions: the evaluating leaf has at most this
 // many points (one pass of four row tiles of 16: each wave holds every target)
@@ -156,6 +159,15 @@ struct KGen {
     int tneg, pad;
 };
 
+// A piece [begin, end) of the operator table's generated part.  Setup makes the pieces one
+// after the other in the same memory: generates its kernel matrices, multiplies, packs.
+struct SetupWindow {
+    int64_t begin, end;
+    int k0, k1;                // KGen jobs
+    int s0, s1;                // setup GEMM stages
+    int p0[2], p1[2];          // PackA jobs, FP64 and FP32
+};
+
 enum StageKind : int {
     ST_ZERO = 0, ST_GATHER, ST_SCATTER, ST_KAPPLY, ST_GEMM, ST_FFTFWD, ST_VLIST, ST_REDUCE,
     ST_FORK,        // the second stream waits for everything issued so far on the first (event buf)
@@ -174,7 +186,7 @@ struct Stage {
     int kind;
     int begin, end;     // descriptor range (tasks / tiles / sources / targets)
     int buf;            // ST_ZERO: buffer id; ST_FORK/ST_JOIN: event index; ST_VLIST: first chunk;
-                        // ST_REDUCE: the contributions' buffer
+                        // ST_REDUCE: the contributions' buffer; setup GEMMs: A's buffer
     int64_t count;      // ST_ZERO: elements per rhs; ST_VLIST: chunks
     int prec;           // StagePrec
     int stream;         // 0: the evaluation (caller's) stream, 1: the concurrent second stream

@@ -16,6 +16,8 @@
 #include "planner.hpp"
 
 #include <algorithm>
+#include <array>
+#include <cstdint>
 #include <set>
 #include <cstring>
 #include <sstream>
@@ -538,6 +540,7 @@ struct Builder {
     void stages_lf_downward();
     void stages_leaf();
     void pack_operators();
+    void setup_windows();
     void finish(bool want_dump);
 
     // Every descriptor's element range must lie inside the buffer or table it indexes: the
@@ -608,19 +611,62 @@ struct Builder {
             need(t.mb >= 1 && t.mb <= GEMM_MB && t.m0 >= 0 && t.m0 % 16 == 0 && t.m0 < g.M &&
                  t.m0 + 16 * (t.mb - 1) < g.M && t.n0 >= 0 && t.n0 < g.ncols, "tile index");
         }
-        auto bsize = [&](int b) { return b == BUF_OPMAT ? pl.opmat_total : pl.bufsize[b]; };
-        for (const Stage& st : pl.setup_stages) {
-            need(st.kind == ST_GEMM && st.begin >= 0 && st.begin <= st.end && st.end <= (int64_t)pl.tiles.size(),
-                 "setup stage");
-            for (int t = st.begin; t < st.end; ++t) {
-                need(pl.tiles[t].mb == st.mb, "setup tile height");
-                const GGroup& g = pl.groups[pl.tiles[t].g];
-                need(g.transA == 0 && st.trans == 0, "setup operand order");
-                need(g.bbuf == BUF_OPMAT && g.cbuf == BUF_OPMAT, "setup buffers");
+        auto bsize = [&](int b) {
+            return b == BUF_OPMAT ? pl.opmat_up : b == BUF_OPGEN ? pl.opmat_total : pl.bufsize[b];
+        };
+        // the windows cover every job, stage and tile of the setup once, in order, and hold what
+        // these read and write of the generated part
+        {
+            int k = 0, s = 0, t1 = pl.setup_t0, pk[2] = {pl.pack_up[0], pl.pack_up[1]};
+            int64_t at = pl.opmat_up;
+            auto pack_end = [](const PackA& p) {
+                return p.src + (p.trans ? (int64_t)(p.M - 1) * p.lda + p.K : (int64_t)(p.K - 1) * p.lda + p.M);
+            };
+            for (int f32 = 0; f32 < 2; ++f32)
+                for (int j = 0; j < pl.pack_up[f32]; ++j) {
+                    const PackA& p = (f32 ? pl.pack32 : pl.pack64)[j];
+                    need(p.src >= 0 && pack_end(p) <= pl.opmat_up, "packed block of the uploaded part");
+                }
+            for (const SetupWindow& w : pl.windows) {
+                need(w.begin >= at && w.begin < w.end && w.end <= pl.opmat_total &&
+                         w.end - w.begin <= pl.window_elems, "setup window");
+                auto in = [&](int64_t b, int64_t n) { return b >= w.begin && b + n <= w.end; };
+                at = w.end;
+                need(w.k0 == k && w.k0 <= w.k1 && w.k1 <= (int)pl.kgen.size(), "setup window kernel matrices");
+                for (; k < w.k1; ++k) need(in(pl.kgen[k].out, (int64_t)pl.kgen[k].m * pl.kgen[k].n), "kernel matrix");
+                need(w.s0 == s && w.s0 <= w.s1 && w.s1 <= (int)pl.setup_stages.size(), "setup window stages");
+                for (; s < w.s1; ++s) {
+                    const Stage& st = pl.setup_stages[s];
+                    need(st.kind == ST_GEMM && st.begin == t1 && st.begin < st.end && st.end <= pl.setup_t1,
+                         "setup stage");
+                    t1 = st.end;
+                    for (int t = st.begin; t < st.end; ++t) {
+                        need(pl.tiles[t].mb == st.mb, "setup tile height");
+                        const GGroup& g = pl.groups[pl.tiles[t].g];
+                        need(g.transA == 0 && g.kb == 0 && g.soff < 0, "setup operand");
+                        need(g.bbuf >= BUF_OPMAT && g.cbuf == BUF_OPGEN && st.buf >= BUF_OPMAT, "setup buffers");
+                        const int64_t na = (int64_t)(g.K - 1) * g.lda + g.M;
+                        need(st.buf == BUF_OPGEN ? in(g.aoff, na) : g.aoff + na <= pl.opmat_up, "setup A");
+                        if (t > st.begin && pl.tiles[t - 1].g == pl.tiles[t].g) continue;
+                        for (int n = 0; n < g.ncols; ++n)
+                            need(in(pl.colC[g.col0 + n], g.M) && (g.bbuf == BUF_OPMAT || in(pl.colB[g.bcol0 + n], g.K)),
+                                 "setup columns");
+                    }
+                }
+                for (int f32 = 0; f32 < 2; ++f32) {
+                    const std::vector<PackA>& jobs = f32 ? pl.pack32 : pl.pack64;
+                    need(w.p0[f32] == pk[f32] && w.p0[f32] <= w.p1[f32] && w.p1[f32] <= (int)jobs.size(),
+                         "setup window packing");
+                    for (int j = w.p0[f32]; j < w.p1[f32]; ++j)
+                        need(in(jobs[j].src, pack_end(jobs[j]) - jobs[j].src), "packed block");
+                    pk[f32] = w.p1[f32];
+                }
             }
+            need(k == (int)pl.kgen.size() && s == (int)pl.setup_stages.size() && t1 == pl.setup_t1 &&
+                     pk[0] == (int)pl.pack64.size() && pk[1] == (int)pl.pack32.size(), "setup windows");
         }
         for (const GGroup& g : pl.groups) {
-            need(g.bbuf >= 0 && g.bbuf <= BUF_OPMAT && g.cbuf >= 0 && g.cbuf <= BUF_OPMAT, "gemm buffers");
+            need(g.bbuf >= 0 && g.bbuf < BUF_ALL && g.cbuf >= 0 && g.cbuf < BUF_ALL, "gemm buffers");
             need(g.col0 >= 0 && g.col0 + (int64_t)g.ncols <= (int64_t)pl.colC.size(), "gemm C columns");
             for (int n = 0; n < g.ncols; ++n) {
                 const int64_t c = pl.colC[g.col0 + n];
@@ -636,11 +682,8 @@ struct Builder {
                 }
                 const int64_t last = g.transA ? aoff + (int64_t)(g.M - 1) * g.lda + kcols
                                               : aoff + (int64_t)(kcols - 1) * g.lda + g.M;
-                // the kernel reads whole row blocks of 16 and up to GEMM_AHEAD past the last k
-                const int64_t mr = (g.M + 15) / 16 * 16, kr = kcols + GEMM_AHEAD;
-                const int64_t read = g.transA ? aoff + (mr - 1) * g.lda + kr : aoff + (kr - 1) * g.lda + mr;
                 return aoff >= 0 && last <= pl.opmat_total && g.lda >= (g.transA ? kcols : g.M) &&
-                       read <= pl.opmat_total + pl.opmat_pad;
+                       last - aoff <= INT32_MAX;      // offsets within a block are 32 bits wide
             };
             if (g.kb == 0) {
                 need(a_ok(g.aoff, g.K), "gemm A");
@@ -1126,7 +1169,7 @@ void Builder::operator_layout() {
                 }
                 GGroup g{};
                 g.aoff = h.e1; g.soff = -1; g.M = h.r1; g.K = h.r2; g.lda = h.r1; g.transA = 0; g.mode = 0;
-                g.bbuf = BUF_OPMAT; g.cbuf = BUF_OPMAT;
+                g.bbuf = BUF_OPGEN; g.cbuf = BUF_OPGEN;
                 add_group(g, bc, cc, nullptr, 0, {}, false);
                 if (lv.first != 1.0) continue;
                 for (int c = 0; c < 8; ++c) {
@@ -1137,17 +1180,12 @@ void Builder::operator_layout() {
                     }
                     GGroup q{};
                     q.aoff = G_(h.de2dc[c]); q.soff = -1; q.M = h.r1c; q.K = h.r2; q.lda = h.r1c; q.transA = 0;
-                    q.mode = 0; q.bbuf = BUF_OPMAT; q.cbuf = BUF_OPMAT;
+                    q.mode = 0; q.bbuf = BUF_OPMAT; q.cbuf = BUF_OPGEN;
                     add_group(q, bd, cd, nullptr, 0, {}, false);
                 }
             }
-        if ((int)pl.tiles.size() > g0) {
-            Stage s;
-            std::memset(&s, 0, sizeof(s));
-            s.kind = ST_GEMM; s.begin = g0; s.end = (int)pl.tiles.size(); s.prec = PREC_SOLVE; s.lstage = -1;
-            std::strncpy(s.name, "setup_fuse", sizeof(s.name) - 1);
-            push_gemm_stages(pl.setup_stages, s);
-        }
+        pl.setup_t0 = g0;
+        pl.setup_t1 = (int)pl.tiles.size();
     }
 }
 
@@ -1817,12 +1855,110 @@ void Builder::pack_operators() {
     pl.pack32_total += slack[1];
 }
 
+// The generated part of the operator table is never in memory whole: an evaluation reads
+// packed blocks, so setup makes it in windows.  A window holds whole units, the shortest
+// runs of the table that no kernel matrix, product or packed block crosses (a direction's
+// child kernels with their products, an M2L matrix).  64 MiB: a window's launches fill the
+// chip and their own times stay small (6k points MIXED: generation, products and packing 1.1 ms;
+// 1.9 at 32 MiB, 3.4 at 16, 0.7 for the whole table).  Under a budget a window with the setup's
+// lists takes no more than one right-hand side's buffers, which come after it, if a unit
+// allows: setup then needs no more than an evaluation.
+void Builder::setup_windows() {
+    constexpr int64_t WINDOW_BYTES = int64_t(64) << 20;
+    const int64_t up = pl.opmat_up;
+    struct Span {
+        int64_t b, e;
+    };
+    std::vector<Span> spans, units;
+    for (const KGen& k : pl.kgen) spans.push_back({k.out, k.out + (int64_t)k.m * k.n});
+    for (int t = pl.setup_t0, last = -1; t < pl.setup_t1; ++t) {
+        if (pl.tiles[t].g == last) continue;
+        last = pl.tiles[t].g;
+        const GGroup& g = pl.groups[last];
+        Span s{INT64_MAX, 0};
+        auto add = [&](int64_t b, int64_t n) {
+            s.b = std::min(s.b, b);
+            s.e = std::max(s.e, b + n);
+        };
+        if (g.aoff >= up) add(g.aoff, (int64_t)(g.K - 1) * g.lda + g.M);
+        for (int n = 0; n < g.ncols; ++n) {
+            if (g.bbuf == BUF_OPGEN) add(pl.colB[g.bcol0 + n], g.K);
+            add(pl.colC[g.col0 + n], g.M);
+        }
+        spans.push_back(s);
+    }
+    std::sort(spans.begin(), spans.end(), [](const Span& x, const Span& y) { return x.b < y.b; });
+    for (const Span& s : spans) {
+        if (!units.empty() && s.b < units.back().e) units.back().e = std::max(units.back().e, s.e);
+        else units.push_back(s);
+    }
+    const int64_t bytes = prm.budget ? std::min(WINDOW_BYTES, pl.rhs_bytes() - pl.setup_bytes()) : WINDOW_BYTES;
+    const int64_t limit = bytes / 16 - GEMM_AHEAD;
+    for (const Span& u : units) {
+        if (pl.windows.empty() || u.e - pl.windows.back().begin > limit) {
+            SetupWindow w{};
+            w.begin = u.b;
+            pl.windows.push_back(w);
+        }
+        SetupWindow& w = pl.windows.back();
+        w.end = u.e;
+        pl.window_elems = std::max(pl.window_elems, w.end - w.begin);
+    }
+    auto window_of = [&](int64_t off) {
+        auto it = std::upper_bound(pl.windows.begin(), pl.windows.end(), off,
+                                   [](int64_t o, const SetupWindow& w) { return o < w.begin; });
+        return (int)(it - pl.windows.begin()) - 1;
+    };
+    // jobs in table order, so that a window's are adjacent
+    std::vector<std::array<int, 3>> key(pl.groups.size());          // of setup groups: window, A's buffer
+    for (int t = pl.setup_t0; t < pl.setup_t1; ++t) {
+        const GGroup& g = pl.groups[pl.tiles[t].g];
+        key[pl.tiles[t].g] = {window_of(pl.colC[g.col0]), g.aoff >= up ? BUF_OPGEN : BUF_OPMAT, 0};
+    }
+    auto tile_key = [&](const GTile& t) {
+        std::array<int, 3> k = key[t.g];
+        k[2] = t.mb;
+        return k;
+    };
+    std::stable_sort(pl.tiles.begin() + pl.setup_t0, pl.tiles.begin() + pl.setup_t1,
+                     [&](const GTile& x, const GTile& y) { return tile_key(x) < tile_key(y); });
+    std::stable_sort(pl.kgen.begin(), pl.kgen.end(), [](const KGen& x, const KGen& y) { return x.out < y.out; });
+    for (int f32 = 0; f32 < 2; ++f32) {
+        std::vector<PackA>& jobs = f32 ? pl.pack32 : pl.pack64;
+        std::stable_sort(jobs.begin(), jobs.end(), [](const PackA& x, const PackA& y) { return x.src < y.src; });
+        while (pl.pack_up[f32] < (int)jobs.size() && jobs[pl.pack_up[f32]].src < up) ++pl.pack_up[f32];
+    }
+    int k = 0, t = pl.setup_t0, p[2] = {pl.pack_up[0], pl.pack_up[1]};
+    for (int i = 0; i < (int)pl.windows.size(); ++i) {
+        SetupWindow& w = pl.windows[i];
+        w.k0 = k;
+        while (k < (int)pl.kgen.size() && pl.kgen[k].out < w.end) ++k;
+        w.k1 = k;
+        w.s0 = (int)pl.setup_stages.size();
+        while (t < pl.setup_t1 && key[pl.tiles[t].g][0] == i) {
+            const std::array<int, 3> q = tile_key(pl.tiles[t]);
+            Stage s;
+            std::memset(&s, 0, sizeof(s));
+            s.kind = ST_GEMM; s.begin = t; s.prec = PREC_SOLVE; s.lstage = -1; s.buf = q[1]; s.mb = q[2];
+            std::strncpy(s.name, "setup_fuse", sizeof(s.name) - 1);
+            while (t < pl.setup_t1 && tile_key(pl.tiles[t]) == q) ++t;
+            s.end = t;
+            pl.setup_stages.push_back(s);
+        }
+        w.s1 = (int)pl.setup_stages.size();
+        for (int f32 = 0; f32 < 2; ++f32) {
+            const std::vector<PackA>& jobs = f32 ? pl.pack32 : pl.pack64;
+            w.p0[f32] = p[f32];
+            while (p[f32] < (int)jobs.size() && jobs[p[f32]].src < w.end) ++p[f32];
+            w.p1[f32] = p[f32];
+        }
+    }
+}
+
 void Builder::finish(bool want_dump) {
     auto& boxes = tree.boxes;
     pack_operators();
-    for (const GGroup& g : pl.groups)
-        if (g.transA < 2)
-            pl.opmat_pad = std::max(pl.opmat_pad, GEMM_AHEAD * (int64_t)g.lda + 16);
+    setup_windows();
     for (const GGroup& g : pl.groups)
         pl.zeros = std::max<int64_t>(pl.zeros, (g.kb ? g.kb : g.K) + GEMM_AHEAD);
     // ---------------- per-stage algorithmic work (per RHS)

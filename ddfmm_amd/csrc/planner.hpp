@@ -44,8 +44,10 @@ struct HostPlan {
     int64_t opmat_up = 0;                  // uploaded part alone
     std::vector<PackA> pack32, pack64;     // operator blocks packed at setup, per table
     int64_t pack32_total = 0, pack64_total = 0;   // with the slack behind them (GEMM_AHEAD)
-    int64_t zeros = 0;                     // length of the GEMMs' block of zeros
-    int64_t opmat_pad = 0;                 // zeros behind the table: the setup GEMMs read whole row blocks and units
+    int64_t zeros = 0;                     // length of the GEMMs' block of zeros, behind the uploaded part
+    std::vector<SetupWindow> windows;      // the generated part, in order
+    int64_t window_elems = 0;              // the longest of them
+    int pack_up[2] = {0, 0};               // packing jobs (FP64, FP32) from the uploaded part: the first ones
     std::vector<int> grid;                 // FFT grid index tables
     std::vector<double> genpts;            // kernel-generation point table (xyz rows)
     std::vector<KGen> kgen;
@@ -63,11 +65,24 @@ struct HostPlan {
     std::vector<int> vpk;                   // packed pairs per target, padded to multiples of 8
     std::vector<RTarget> rtrg;
     std::vector<Stage> stages;
-    std::vector<Stage> setup_stages;       // FP64 GEMMs on the operator table, run once after generation
+    std::vector<Stage> setup_stages;       // FP64 GEMMs on the operator table, window by window
+    int setup_t0 = 0, setup_t1 = 0;        // their tiles
     std::vector<LogicalGemm> lgemm;        // logical GEMM stages of `stages` (Stage::lstage)
     int64_t bufsize[BUF_COUNT] = {0};      // elements per rhs
     PlanStats stats;
     std::string dump;                      // canonical text of the lists (debug/parity)
+
+    int64_t vector_bytes() const { return prm.xlat > 0 ? 8 : 16; }    // of a work buffer's element
+    int64_t rhs_bytes() const {            // work buffers and staging of one right-hand side
+        int64_t n = 0;
+        for (int64_t b : bufsize) n += b;
+        return 2 * N * 16 + n * vector_bytes();
+    }
+    // what setup holds besides the tables it leaves and the window
+    int64_t setup_bytes() const {
+        return (int64_t)(genpts.size() * sizeof(double) + kgen.size() * sizeof(KGen) +
+                         (pack32.size() + pack64.size()) * sizeof(PackA));
+    }
 };
 
 void build_plan(const Params& prm, const double* pos, int64_t N, const Mlib& mlib,

@@ -107,6 +107,7 @@ void retile(HostPlan& pl, const std::vector<int>& mbmax) {
     pl.tiles.swap(tiles);
     pl.stages.swap(stages);
     pl.setup_stages.clear();
+    pl.windows.clear();
     for (Stage& s : pl.stages) stage_work(pl, s);
 }
 

@@ -234,8 +234,8 @@ class Wave3d:
 
     def memory(self) -> dict:
         """Device bytes of the set-up context (ddfmm_memory): tables, one right-hand side's
-        work buffers and staging, setup-only generator tables, and the right-hand sides
-        per pass under the HBM budget."""
+        work buffers and staging, setup-only tables, and the right-hand sides per pass under
+        the HBM budget."""
         f, r, t, s = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int()
         check(lib().ddfmm_memory(self._ctx, ctypes.byref(f), ctypes.byref(r), ctypes.byref(t), ctypes.byref(s)))
         return {"fixed_bytes": f.value, "per_rhs_bytes": r.value, "setup_bytes": t.value, "slab": s.value}

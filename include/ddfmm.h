@@ -133,9 +133,9 @@ DDFMM_API int ddfmm_get_tiles(ddfmm_ctx* ctx, int cap, int* mbmax, char* names /
    more right-hand sides run in passes of `slab`; results are the same bits as in one
    pass.  Setup fails with DDFMM_ENOMEM, naming the minimum, when not even one
    right-hand side fits.  ddfmm_memory reports the device bytes of the tables (fixed),
-   of one right-hand side's work buffers and staging (per_rhs), of the setup-only
-   generator tables (setup) and the slab; also on host-only contexts, where it is the
-   plan's requirement. */
+   of one right-hand side's work buffers and staging (per_rhs), of what lives during setup
+   only (setup: generator tables and the piece of the operator table being made) and the
+   slab; also on host-only contexts, where it is the plan's requirement. */
 DDFMM_API int ddfmm_set_hbm_budget(ddfmm_ctx* ctx, int64_t bytes);
 DDFMM_API int ddfmm_memory(ddfmm_ctx* ctx, int64_t* fixed_bytes, int64_t* per_rhs_bytes, int64_t* setup_bytes,
                            int* slab);

@@ -78,3 +78,27 @@ for p in (FP64, MIXED, FP64_FUSED, MIXED_SPLIT):
         assert hip.host_hip_live() == 0, (p, i, n, hip.host_hip_live())
     print("precision", p, "calls", n, flush=True)
 """)
+
+
+def test_operator_tables_after_setup(run):
+    """A context keeps the packed operators and the uploaded part of the table, not the table
+    itself; the reported bytes are what is allocated.  A budget of the tables and one
+    right-hand side is enough for the setup too."""
+    run("""
+for p in (FP64, MIXED, FP64_FUSED, MIXED_SPLIT):
+    w = wave(p, nrhs=2, k=4.0, n=6000)
+    m, st = w.memory(), w.stats()
+    table = 16 * st["opmat_elems"]
+    print("precision", p, m, "table", table, "live", hip.host_hip_live(), flush=True)
+    assert hip.host_hip_live() == st["device_bytes"] == m["fixed_bytes"] + 2 * m["per_rhs_bytes"]
+    # against the table itself (beside it, the packed blocks made these 2.06, 1.29, 1.54 and 2.51)
+    assert m["fixed_bytes"] < {FP64: 1.2, MIXED: 0.4, FP64_FUSED: 0.7, MIXED_SPLIT: 1.2}[p] * table, p
+    w.close()
+    hip.host_hip_reset()
+    budget = m["fixed_bytes"] + m["per_rhs_bytes"] + 1024
+    w = wave(p, nrhs=2, k=4.0, n=6000, budget=budget)
+    b = w.memory()
+    print("  budget", budget, b, "peak", hip.host_hip_peak(), flush=True)
+    assert b["slab"] == 1 and b["fixed_bytes"] + b["per_rhs_bytes"] <= budget and hip.host_hip_peak() <= budget
+    w.close()
+""")
