@@ -131,27 +131,6 @@ struct SetupTable {
     SetupTable& operator=(const SetupTable&) = delete;
 };
 
-// Device bytes of a set-up context: `fixed` for the point, operator and descriptor
-// tables (kept for the context's life), `per_rhs` for the work buffers and the staging
-// of one right-hand side, `transient` for what lives only during setup (freed before the
-// work buffers are allocated): the window of the operator table's generated part that is
-// being made, the generator tables and the packing jobs.
-template <class T>
-static int64_t vbytes(const std::vector<T>& v) { return (int64_t)v.size() * (int64_t)sizeof(T); }
-static void plan_bytes(const HostPlan& h, int precision, int64_t& fixed, int64_t& per_rhs, int64_t& transient) {
-    const bool mixed = precision == DDFMM_MIXED || precision == DDFMM_MIXED_SPLIT;
-    fixed = vbytes(h.px) + vbytes(h.py) + vbytes(h.pz) + 2 * vbytes(h.perm) + vbytes(h.grid) +
-            (h.opmat_up + h.zeros) * (int64_t)sizeof(double2) + (mixed ? h.opmat_up * (int64_t)sizeof(float2) : 0) +
-            h.pack32_total * (int64_t)sizeof(float2) + h.pack64_total * (int64_t)sizeof(double2) +
-            (precision == DDFMM_MIXED_SPLIT ? h.opmat_total * 16 : 0) +
-            vbytes(h.ktasks) + vbytes(h.ksrcs) + vbytes(h.groups) + vbytes(h.tiles) + vbytes(h.colB) +
-            vbytes(h.colC) + vbytes(h.colA) + vbytes(h.fsrc) + vbytes(h.vtrg) + vbytes(h.vchunk) +
-            vbytes(h.vsrc) + vbytes(h.vpk) + vbytes(h.rtrg) + (int64_t)sizeof(IoPtrs);
-    per_rhs = h.rhs_bytes();
-    for (int b = 0; b < BUF_COUNT; ++b) fixed += h.bufsize[b] > 0 ? BUF_SLACK * h.vector_bytes() : 0;
-    transient = h.setup_bytes() + (h.windows.empty() ? 0 : (h.window_elems + GEMM_AHEAD) * (int64_t)sizeof(double2));
-}
-
 // The kernel-apply flavour is fixed per context (each right-hand side then has the same
 // bits alone and in any batch): the matrix-core kernel in the mixed modes from four
 // right-hand sides up, the vector-ALU kernel otherwise.
@@ -288,6 +267,12 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         // reduction of the mirror products costs more than it saves)
         q.near_pairs = kapply_on_mfma(p->precision, p->nrhs_max) && p->ptsmax <= 2 * MIRROR_MAX_TARGETS;
         q.budget = c->hbm_budget > 0;
+        q.room = c->hbm_budget;
+        if (!q.budget && c->device >= 0) {
+            size_t free = 0, total = 0;
+            HIPCHK(hipMemGetInfo(&free, &total));
+            q.room = (int64_t)free;
+        }
         c->nrhs_max = p->nrhs_max;
         c->precision = p->precision;
         std::shared_ptr<const Mlib> mlib = shared ? shared : load_mlib(ldfile, hdfile);
@@ -300,7 +285,10 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
     // HBM budget: the work buffers hold `slab` right-hand sides; an evaluation of more
     // runs in passes of at most `slab` (each right-hand side is independent, so the
     // results are the same bits as in one pass).
-    plan_bytes(c->hp, c->precision, c->fixed_bytes, c->rhs_bytes, c->setup_transient);
+    const PlanBytes bytes = plan_bytes(c->hp);
+    c->fixed_bytes = bytes.fixed;
+    c->rhs_bytes = bytes.per_rhs;
+    c->setup_transient = bytes.setup;
     c->slab = c->nrhs_max;
     if (c->hbm_budget > 0) {
         const int64_t need = c->fixed_bytes + std::max(c->rhs_bytes, c->setup_transient);
@@ -335,10 +323,11 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         d.grid = c->upload(h.grid);
         // the window's memory first and, without a budget, given back last: taken after the
         // large tables, or freed before the work buffers, it cost 2 ms of a setup of 13
-        auto window = std::make_unique<SetupTable<double2>>(h.windows.empty() ? 0 : h.window_elems + GEMM_AHEAD);
-        // uploaded part of the operator table, the GEMMs' zeros behind it
-        d.opmat = c->alloc<double2>(h.opmat_up + h.zeros);
-        d.zeros = d.opmat + h.opmat_up;
+        auto window = std::make_unique<SetupTable<double2>>(h.stored || h.windows.empty() ? 0 : h.window_elems + GEMM_AHEAD);
+        // operator table (its uploaded part, unless the GEMMs read it), the GEMMs' zeros behind it
+        const int64_t kept = h.stored ? h.opmat_total : h.opmat_up;
+        d.opmat = c->alloc<double2>(kept + h.zeros);
+        d.zeros = d.opmat + kept;
         if (h.zeros > 0) HIPCHK(hipMemset(d.zeros, 0, (size_t)h.zeros * sizeof(double2)));
         if (!h.opmat.empty())
             HIPCHK(hipMemcpy(d.opmat, h.opmat.data(), h.opmat.size() * sizeof(double2), hipMemcpyHostToDevice));
@@ -371,12 +360,12 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
             };
             const int none[2] = {0, 0};
             pack(d.opmat, none, h.pack_up);
-            // the generated part, one window after the other in the same memory: kernel
-            // matrices, fused operators (solves folded into the translations by FP64 GEMMs),
+            // the generated part, one window after the other in the same memory (or in the
+            // table itself): kernel matrices, fused operators (solves folded into the translations by FP64 GEMMs),
             // packed blocks
             d.bt.p[BUF_OPMAT] = d.opmat;
             for (const SetupWindow& w : h.windows) {
-                double2* gen = window->p - w.begin;     // indexed by table offsets of the window
+                double2* gen = h.stored ? d.opmat : window->p - w.begin;   // indexed by table offsets
                 d.bt.p[BUF_OPGEN] = gen;
                 HIPCHK(launch_kgen(kgen.p + w.k0, w.k1 - w.k0, gp.p, gen, d.ktype, c->stream));
                 for (int q = w.s0; q < w.s1; ++q) HIPCHK(launch_setup_gemm(d, h.setup_stages[q], c->stream));
@@ -394,8 +383,7 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
             const int64_t n = h.bufsize[b] > 0 ? h.bufsize[b] * c->slab + BUF_SLACK : 0;
             d.bt.p[b] = esz == 8 ? (void*)c->alloc<float2>(n) : (void*)c->alloc<double2>(n);
         }
-        d.den_io = c->alloc<double2>(h.N * c->slab);
-        d.val_io = c->alloc<double2>(h.N * c->slab);
+        d.host_io = c->alloc<double2>(h.N * c->slab);
         // host copies no longer needed on the device path
         std::vector<cpx>().swap(h.opmat);
         std::vector<double>().swap(h.genpts);
@@ -508,9 +496,9 @@ int ddfmm_eval(ddfmm_ctx* c, const double* den, double* val, int nrhs) {
             const size_t bytes = (size_t)c->hp.N * nr * sizeof(double2);
             const size_t off = (size_t)c->hp.N * r0 * 2;
             if (c->done_recorded) HIPCHK(hipStreamWaitEvent(c->stream, c->done_ev, 0));
-            HIPCHK(hipMemcpyAsync(c->dp.den_io, den + off, bytes, hipMemcpyHostToDevice, c->stream));
-            run_eval(c, c->dp.den_io, c->dp.val_io, nr, c->stream);
-            HIPCHK(hipMemcpyAsync(val + off, c->dp.val_io, bytes, hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(hipMemcpyAsync(c->dp.host_io, den + off, bytes, hipMemcpyHostToDevice, c->stream));
+            run_eval(c, c->dp.host_io, c->dp.host_io, nr, c->stream);
+            HIPCHK(hipMemcpyAsync(val + off, c->dp.host_io, bytes, hipMemcpyDeviceToHost, c->stream));
         }
         HIPCHK(hipStreamSynchronize(c->stream));
     } catch (const std::exception& e) {
@@ -577,7 +565,7 @@ static std::vector<double> time_logical(ddfmm_ctx* c, int nrhs, int reps) {
         c->ev.assign(2 * stages.size(), nullptr);
         for (auto& e : c->ev) HIPCHK(hipEventCreate(&e));
     }
-    HIPCHK(launch_set_io(c->dp.io, c->dp.den_io, c->dp.val_io, c->stream));
+    HIPCHK(launch_set_io(c->dp.io, c->dp.host_io, c->dp.host_io, c->stream));
     for (int r = 0; r <= reps; ++r) {            // the first run warms up
         issue_stages(c, nrhs, c->stream, true, true);
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -606,7 +594,7 @@ int ddfmm_autotune(ddfmm_ctx* c, int nrhs, int reps, int cap, int* mbmax, int* c
     try {
         HIPCHK(hipSetDevice(c->device));
         if (c->done_recorded) HIPCHK(hipStreamWaitEvent(c->stream, c->done_ev, 0));
-        HIPCHK(hipMemsetAsync(c->dp.den_io, 0, (size_t)c->hp.N * nrhs * sizeof(double2), c->stream));
+        HIPCHK(hipMemsetAsync(c->dp.host_io, 0, (size_t)c->hp.N * nrhs * sizeof(double2), c->stream));
         std::vector<int> cur(nl);
         for (int l = 0; l < nl; ++l) cur[l] = c->hp.lgemm[l].mbmax;
         // the planner's tiling (height limit GEMM_MB, rows split further for small stages)

@@ -30,10 +30,10 @@ struct DevPlan {
     int* perm = nullptr;           // sorted position -> input index
     int* iperm = nullptr;          // input index -> sorted position
     int* grid = nullptr;
-    double2* opmat = nullptr;      // uploaded part of the operator table
-    float2* opmat32 = nullptr;     // FP32 copy of it (mixed modes)
+    double2* opmat = nullptr;      // operator table: its uploaded part, or all of it where nothing is packed
+    float2* opmat32 = nullptr;     // FP32 copy of the uploaded part (mixed modes)
     float2* oppack = nullptr;      // packed operator blocks of the GEMMs: FP32 (MIXED translations)
-    double2* oppack64 = nullptr;   // and FP64 (every other GEMM but the split-BF16 ones)
+    double2* oppack64 = nullptr;   // and FP64 (every other GEMM but the split-BF16 ones; null: read as stored)
     double2* zeros = nullptr;      // what the GEMMs read as absent blocks of B
     void* opmatbf = nullptr;       // split-BF16 copy of the whole table (16 bytes per entry; mixed-split mode)
     KTask* ktasks = nullptr;
@@ -48,8 +48,8 @@ struct DevPlan {
     int* vpk = nullptr;
     RTarget* rtrg = nullptr;
     BufTable bt{};
-    double2* den_io = nullptr;     // context-owned [rhs][N] staging of the host-buffer entry point
-    double2* val_io = nullptr;
+    double2* host_io = nullptr;    // context-owned [rhs][N] staging of the host-buffer entry point: the
+                                   // densities, read by the first stage, then the potentials, written by the last
     IoPtrs* io = nullptr;          // device copy of the current evaluation's buffers
 };
 

@@ -56,6 +56,7 @@ struct Params {
     bool fuse_solves = false;   // apply check->equivalent solves as single precomputed matrices
     int nrhs_max = 1;           // right-hand sides an evaluation may carry (GEMM launch sizing)
     bool budget = false;        // device memory is bounded: setup needs no more than one right-hand side
+    int64_t room = 0;           // device bytes for the context (the budget, or what is free); 0: not known
     int xlat = 0;               // translation GEMMs: 0 FP64, 1 FP32, 2 split-BF16 (operators as stored)
     bool near_pairs = false;    // near field: evaluate each pair of leaves that are in each
                                 // other's near lists once, for both directions

@@ -718,7 +718,7 @@ __device__ __forceinline__ CPair load_pair(const float2* p) {
 constexpr int gemm_units(int mb, int cb) { return cb > 1 || mb > 3 ? 1 : mb > 1 ? 2 : 4; }
 
 // PACK: A packed (PackA in plan.hpp) in the order the lanes take it; else as stored in the
-// operator table (the setup's products).
+// operator table (the setup's products, FP64 contexts whose budget holds no packed copy).
 template <class TA, class V, class R, int MB, int CB, bool PACK, bool G3M>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(
     const GGroup* __restrict__ groups, const GTile* __restrict__ tiles,
@@ -788,18 +788,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         }
         wave_lds_order();
     }
-    // A elements of this lane within a unit, per row block and per unit.  As stored, rows
-    // past the group's last repeat that one, and k past the segment's end its first.
+    // A elements of this lane within a unit, per row block and per unit.  As stored (either
+    // order), rows past the group's last repeat that one, and k past the segment's end its
+    // first.
     static_assert(PACK || sizeof(R) == 8, "operators as stored in FP64 only");
     constexpr unsigned ROWS = 64 * UQ;
     const unsigned lda = g.lda;
-    const unsigned ustep = PACK ? ROWS * lda : UK * lda;
+    const unsigned kst = g.transA == 1 ? 1 : lda, ustep = PACK ? ROWS * lda : UK * kst;
     unsigned ao[PACK ? 1 : MB];
     if constexpr (PACK) {
         ao[0] = UQ * lane;
     } else {
 #pragma unroll
-        for (int a = 0; a < MB; ++a) ao[a] = min(tl.m0 + 16 * a + li, g.M - 1);
+        for (int a = 0; a < MB; ++a) ao[a] = min(tl.m0 + 16 * a + li, g.M - 1) * (g.transA == 1 ? lda : 1);
     }
 
     // G3M (FP32 contexts of the e^{ikr}/r kernel): three real products per complex one,
@@ -874,7 +875,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
             }
             const int left = kl - u * UK;          // k left from the unit's first
             const TA* ap = PACK ? Ap + u * ustep + ao[0]
-                                : Ap + ((left > 0 ? u * ustep : 0) + (lk < left ? lk * lda : 0));
+                                : Ap + ((left > 0 ? u * ustep : 0) + (lk < left ? lk * kst : 0));
 #pragma unroll
             for (int a = 0; a < MB; ++a) {
                 if constexpr (PACK && sizeof(R) == 4) {
@@ -1019,6 +1020,12 @@ void launch_gemm_form(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d
         DDFMM_GEMM_MB(6) DDFMM_GEMM_MB(7)
     }
 #undef DDFMM_GEMM_MB
+}
+
+// FP64 products, on packed operators or, where the context holds none, as stored.
+void launch_gemm64(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
+    if (d.oppack64) launch_gemm_form<double2, double2, double, 1, true, false>(s, nrhs, st, d, d.oppack64);
+    else launch_gemm_form<double2, double2, double, 1, false, false>(s, nrhs, st, d, d.opmat);
 }
 
 // FP32 products on packed operators.  Two column blocks per wave (CB = 2) halve the operator
@@ -2004,7 +2011,7 @@ hipError_t launch_stage_t(const DevPlan& d, const Stage& s, int nrhs, hipStream_
         else if (d.mixed)
             launch_gemm32<false>(s, nrhs, st, d);
         else
-            launch_gemm_form<double2, double2, double, 1, true, false>(s, nrhs, st, d, d.oppack64);
+            launch_gemm64(s, nrhs, st, d);
         break;
     case ST_FFTFWD:
         if (d.P != 6) return hipErrorInvalidValue;

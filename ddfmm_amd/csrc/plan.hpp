@@ -195,7 +195,6 @@ struct Stage {
     int mb;             // ST_GEMM: row blocks of every tile in the range (one kernel instance);
                         // ST_KAPPLY: 1 when sources carry mirror slots (KSrc::moff)
     int lstage;         // ST_GEMM: logical stage (all tile heights of one planned GEMM stage), else -1
-    int trans;          // ST_GEMM: transA of every group in the range
     int kblocked;       // ST_GEMM: the groups' K is blocked (GGroup::kb > 0)
     double exec;        // ST_GEMM: MFMA flops per RHS the kernel executes (padding included)
     char name[24];

@@ -333,7 +333,6 @@ struct Builder {
             if (pl.tiles[t].mb < 1 || pl.tiles[t].mb > GEMM_MB) throw Error("internal: tile height out of range");
             Stage q = s;
             q.begin = t; q.end = u; q.mb = pl.tiles[t].mb;
-            q.trans = pl.groups[pl.tiles[t].g].transA;
             q.kblocked = pl.groups[pl.tiles[t].g].kb > 0;
             dst.push_back(q);
             t = u;
@@ -539,8 +538,10 @@ struct Builder {
     void stages_hf_downward();
     void stages_lf_downward();
     void stages_leaf();
-    void pack_operators();
+    std::map<std::pair<int64_t, int>, PackA> packs[2];      // FP64, FP32: (table offset, order) -> block
+    void pack_operators(bool rewrite);
     void setup_windows();
+    void choose_operators();
     void finish(bool want_dump);
 
     // Every descriptor's element range must lie inside the buffer or table it indexes: the
@@ -556,9 +557,11 @@ struct Builder {
             need(st.begin >= 0 && st.begin <= st.end, "stage range");
             if (st.kind == ST_GEMM) {
                 need(st.end <= (int64_t)pl.tiles.size(), "gemm stage");
+                const int form = pl.gemm_form(st);
                 for (int t = st.begin; t < st.end; ++t) {
                     need(pl.tiles[t].mb == st.mb, "gemm stage tile height");
-                    need(pl.groups[pl.tiles[t].g].transA == st.trans, "gemm stage operand order");
+                    const int order = pl.groups[pl.tiles[t].g].transA;
+                    need(form ? order == form : order == 0 || order == 1, "gemm stage operand order");
                 }
             }
             if (st.kind == ST_KAPPLY) need(st.end <= (int64_t)pl.ktasks.size(), "kapply stage");
@@ -1808,45 +1811,43 @@ void Builder::stages_leaf() {
 }
 
 // Packed copies of the operator blocks that the evaluation's GEMMs read (each block once per
-// table and operand order); their groups then point into the packed tables.
-void Builder::pack_operators() {
-    std::map<std::pair<int64_t, int>, int> done[2];       // FP32, FP64: (table offset, order) -> job
+// table and operand order): lists them, or with `rewrite` points the groups to them.
+void Builder::pack_operators(bool rewrite) {
     auto packed = [&](bool f32, int64_t off, int K, const GGroup& g) {
-        std::vector<PackA>& jobs = f32 ? pl.pack32 : pl.pack64;
-        int64_t& total = f32 ? pl.pack32_total : pl.pack64_total;
-        auto it = done[f32].find({off, g.transA});
-        if (it != done[f32].end()) {
-            const PackA& p = jobs[it->second];
-            if (p.M != g.M || p.K != K || p.lda != g.lda) throw Error("internal: operator block packed in two shapes");
-            return p.dst;
+        auto it = packs[f32].find({off, g.transA});
+        if (it == packs[f32].end()) {
+            int64_t& total = f32 ? pl.pack32_total : pl.pack64_total;
+            PackA p{};
+            p.src = off; p.dst = total; p.M = g.M; p.K = K; p.lda = g.lda; p.trans = g.transA;
+            total += pack_elems(f32, g.M, K);
+            (f32 ? pl.pack32 : pl.pack64).push_back(p);
+            it = packs[f32].insert({{off, g.transA}, p}).first;
         }
-        PackA p{};
-        p.src = off; p.dst = total; p.M = g.M; p.K = K; p.lda = g.lda; p.trans = g.transA;
-        total += pack_elems(f32, g.M, K);
-        done[f32][{off, g.transA}] = (int)jobs.size();
-        jobs.push_back(p);
+        const PackA& p = it->second;
+        if (p.M != g.M || p.K != K || p.lda != g.lda) throw Error("internal: operator block packed in two shapes");
         return p.dst;
     };
     std::vector<char> seen(pl.groups.size(), 0);
     for (Stage& st : pl.stages) {
-        if (st.kind != ST_GEMM || (st.prec == PREC_TRANSLATION && prm.xlat == 2)) continue;
-        const bool f32 = st.prec == PREC_TRANSLATION && prm.xlat == 1;
+        const int form = pl.gemm_form(st);
+        if (st.kind != ST_GEMM || form == 0) continue;
         for (int t = st.begin; t < st.end; ++t) {
             if (seen[pl.tiles[t].g]) continue;
             seen[pl.tiles[t].g] = 1;
             GGroup& g = pl.groups[pl.tiles[t].g];
+            const bool f32 = form == 2;
             if (f32 && g.soff >= 0) throw Error("internal: row scale on an FP32 operator");
-            if (g.kb == 0) {
-                g.aoff = packed(f32, g.aoff, g.K, g);
-            } else {
-                for (int h = 0; h < g.K / g.kb; ++h)
-                    pl.colA[g.acol0 + h] = packed(f32, pl.colA[g.acol0 + h], g.kb, g);
+            for (int h = 0; h < (g.kb ? g.K / g.kb : 1); ++h) {
+                int64_t& off = g.kb ? pl.colA[g.acol0 + h] : g.aoff;
+                const int64_t dst = packed(f32, off, g.kb ? g.kb : g.K, g);
+                if (rewrite) off = dst;
             }
+            if (!rewrite) continue;
             g.lda = (g.M + 15) / 16;
-            g.transA = f32 ? 2 : 3;
+            g.transA = form;
         }
-        st.trans = f32 ? 2 : 3;
     }
+    if (rewrite) return;
     int64_t slack[2] = {0, 0};
     for (int f32 = 0; f32 < 2; ++f32)
         for (const PackA& p : f32 ? pl.pack32 : pl.pack64)
@@ -1855,8 +1856,35 @@ void Builder::pack_operators() {
     pl.pack32_total += slack[1];
 }
 
-// The generated part of the operator table is never in memory whole: an evaluation reads
-// packed blocks, so setup makes it in windows.  A window holds whole units, the shortest
+// Packed FP64 operators take up to 1.6 times the table's memory, since a block read in both
+// orders is packed twice.  The GEMMs read the operators as stored instead, with the same bits,
+// where the device's memory (Params::room) holds so many fewer right-hand sides with packed
+// ones that passes of one are left (or none): a pass of one costs more than half of a pass of
+// three (60k points 1.46 and 2.78 ms), reading as stored 6% (60k x 1 1.42 -> 1.51 ms, 6k x 1 0.37 ->
+// 0.39).  Two right-hand sides and more stay packed.
+void Builder::choose_operators() {
+    if (prm.xlat != 0 || prm.room <= 0) return;
+    auto fits = [&]() {            // right-hand sides of a pass
+        const PlanBytes b = plan_bytes(pl);
+        if (prm.budget && b.fixed + std::max(b.per_rhs, b.setup) > prm.room) return int64_t(0);
+        const int64_t beside = b.fixed + (prm.budget ? 0 : b.setup);
+        return std::min<int64_t>(prm.nrhs_max, std::max<int64_t>(0, prm.room - beside) / b.per_rhs);
+    };
+    const int64_t packed = fits();
+    if (packed >= (prm.budget ? std::min(2, prm.nrhs_max) : prm.nrhs_max)) return;
+    pl.stored = true;
+    if (fits() <= packed) {
+        pl.stored = false;
+        return;
+    }
+    pl.pack64.clear();
+    pl.pack64_total = 0;
+    pl.pack_up[0] = 0;
+    for (SetupWindow& w : pl.windows) w.p0[0] = w.p1[0] = 0;
+}
+
+// The generated part of the operator table is not in memory whole where an evaluation reads
+// packed blocks: setup makes it in windows.  A window holds whole units, the shortest
 // runs of the table that no kernel matrix, product or packed block crosses (a direction's
 // child kernels with their products, an M2L matrix).  64 MiB: a window's launches fill the
 // chip and their own times stay small (6k points MIXED: generation, products and packing 1.1 ms;
@@ -1957,10 +1985,12 @@ void Builder::setup_windows() {
 
 void Builder::finish(bool want_dump) {
     auto& boxes = tree.boxes;
-    pack_operators();
-    setup_windows();
     for (const GGroup& g : pl.groups)
         pl.zeros = std::max<int64_t>(pl.zeros, (g.kb ? g.kb : g.K) + GEMM_AHEAD);
+    pack_operators(false);
+    setup_windows();
+    choose_operators();
+    pack_operators(true);
     // ---------------- per-stage algorithmic work (per RHS)
     for (auto& st : pl.stages) stage_work(pl, st);
 
@@ -2007,5 +2037,21 @@ void build_plan(const Params& prm, const double* pos, int64_t N, const Mlib& mli
 }
 
 void validate_plan(const HostPlan& plan) { Builder::validate(plan); }
+
+PlanBytes plan_bytes(const HostPlan& h) {
+    auto bytes = [](const auto& v) { return (int64_t)(v.size() * sizeof(v[0])); };
+    constexpr int64_t C64 = 16, C32 = 8;       // complex values
+    PlanBytes b;
+    b.fixed = bytes(h.px) + bytes(h.py) + bytes(h.pz) + 2 * bytes(h.perm) + bytes(h.grid) +
+              ((h.stored ? h.opmat_total : h.opmat_up) + h.zeros) * C64 + (h.prm.xlat > 0 ? h.opmat_up * C32 : 0) +
+              (h.stored ? 0 : h.pack32_total * C32 + h.pack64_total * C64) +
+              (h.prm.xlat == 2 ? h.opmat_total * 16 : 0) + bytes(h.ktasks) + bytes(h.ksrcs) + bytes(h.groups) +
+              bytes(h.tiles) + bytes(h.colB) + bytes(h.colC) + bytes(h.colA) + bytes(h.fsrc) + bytes(h.vtrg) +
+              bytes(h.vchunk) + bytes(h.vsrc) + bytes(h.vpk) + bytes(h.rtrg) + (int64_t)(2 * sizeof(void*));
+    for (int64_t n : h.bufsize) b.fixed += n > 0 ? BUF_SLACK * h.vector_bytes() : 0;
+    b.per_rhs = h.rhs_bytes();
+    b.setup = h.setup_bytes() + (h.stored || h.windows.empty() ? 0 : (h.window_elems + GEMM_AHEAD) * C64);
+    return b;
+}
 
 }  // namespace ddfmm

@@ -45,6 +45,7 @@ struct HostPlan {
     std::vector<PackA> pack32, pack64;     // operator blocks packed at setup, per table
     int64_t pack32_total = 0, pack64_total = 0;   // with the slack behind them (GEMM_AHEAD)
     int64_t zeros = 0;                     // length of the GEMMs' block of zeros, behind the uploaded part
+    bool stored = false;                   // FP64: the GEMMs read the table itself, nothing is packed
     std::vector<SetupWindow> windows;      // the generated part, in order
     int64_t window_elems = 0;              // the longest of them
     int pack_up[2] = {0, 0};               // packing jobs (FP64, FP32) from the uploaded part: the first ones
@@ -76,17 +77,32 @@ struct HostPlan {
     int64_t rhs_bytes() const {            // work buffers and staging of one right-hand side
         int64_t n = 0;
         for (int64_t b : bufsize) n += b;
-        return 2 * N * 16 + n * vector_bytes();
+        return N * 16 + n * vector_bytes();
     }
     // what setup holds besides the tables it leaves and the window
     int64_t setup_bytes() const {
         return (int64_t)(genpts.size() * sizeof(double) + kgen.size() * sizeof(KGen) +
-                         (pack32.size() + pack64.size()) * sizeof(PackA));
+                         (stored ? 0 : pack32.size() + pack64.size()) * sizeof(PackA));
+    }
+    // GGroup::transA of a stage's groups: 2 or 3 packed, 0 as stored (in either order)
+    int gemm_form(const Stage& s) const {
+        const bool translation = s.prec == PREC_TRANSLATION;
+        return stored || (translation && prm.xlat == 2) ? 0 : translation && prm.xlat == 1 ? 2 : 3;
     }
 };
 
 void build_plan(const Params& prm, const double* pos, int64_t N, const Mlib& mlib,
                 HostPlan& plan, bool want_dump);
+
+// Device bytes of a set-up context: `fixed` for the point, operator and descriptor tables
+// (kept for the context's life), `per_rhs` for the work buffers and the staging of one
+// right-hand side, `setup` for what lives during setup only (under a budget freed before the
+// work buffers are allocated): the window of the operator table's generated part that is
+// being made, the generator tables and the packing jobs.
+struct PlanBytes {
+    int64_t fixed = 0, per_rhs = 0, setup = 0;
+};
+PlanBytes plan_bytes(const HostPlan& plan);
 
 // Throws unless every descriptor's range lies inside the buffer or table it indexes
 // (build_plan ends with it).

@@ -131,7 +131,9 @@ DDFMM_API int ddfmm_get_tiles(ddfmm_ctx* ctx, int cap, int* mbmax, char* names /
    0 = none), setup sizes the work buffers for the largest right-hand-side count `slab`
    (<= nrhs_max) that fits beside the tables, and ddfmm_eval / ddfmm_eval_device with
    more right-hand sides run in passes of `slab`; results are the same bits as in one
-   pass.  Setup fails with DDFMM_ENOMEM, naming the minimum, when not even one
+   pass.  DDFMM_FP64 keeps its operators as stored, with the same results, where packed
+   ones would leave passes of one right-hand side or none (also without a budget, where
+   the free device memory does not hold packed ones).  Setup fails with DDFMM_ENOMEM, naming the minimum, when not even one
    right-hand side fits.  ddfmm_memory reports the device bytes of the tables (fixed),
    of one right-hand side's work buffers and staging (per_rhs), of what lives during setup
    only (setup: generator tables and the piece of the operator table being made) and the

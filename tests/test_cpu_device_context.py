@@ -94,11 +94,47 @@ for p in (FP64, MIXED, FP64_FUSED, MIXED_SPLIT):
     # against the table itself (beside it, the packed blocks made these 2.06, 1.29, 1.54 and 2.51)
     assert m["fixed_bytes"] < {FP64: 1.2, MIXED: 0.4, FP64_FUSED: 0.7, MIXED_SPLIT: 1.2}[p] * table, p
     w.close()
+    w = wave(p, nrhs=1, k=4.0, n=6000)
+    m = w.memory()
+    w.close()
     hip.host_hip_reset()
     budget = m["fixed_bytes"] + m["per_rhs_bytes"] + 1024
-    w = wave(p, nrhs=2, k=4.0, n=6000, budget=budget)
+    w = wave(p, nrhs=1, k=4.0, n=6000, budget=budget)
     b = w.memory()
     print("  budget", budget, b, "peak", hip.host_hip_peak(), flush=True)
     assert b["slab"] == 1 and b["fixed_bytes"] + b["per_rhs_bytes"] <= budget and hip.host_hip_peak() <= budget
     w.close()
+""")
+
+
+def test_operators_as_stored_where_packed_ones_do_not_fit(run):
+    """FP64 contexts fit every budget that held the operator table as stored (the smallest
+    ones of 6000 points on the sphere, before the operators were packed) and whatever memory
+    is free; setup stays within both."""
+    run("""
+least = {FP64: 465267424, MIXED: 1211094528, FP64_FUSED: 826695712, MIXED_SPLIT: 2006617792}
+for p, budget in least.items():
+    w = Wave3d()
+    w.posptr, w.mlibptr = geometry.sphere(6000, 4.0, 1), ml
+    hip.host_hip_reset()
+    w.setup({"-wave3d_ACCU": 2, "-wave3d_K": 4.0, "-wave3d_maxlevel": 14, "-wave3d_hbm_budget": budget / 2**30},
+            nrhs_max=1, precision=p)
+    print("precision", p, "budget", budget, w.memory(), "peak", hip.host_hip_peak(), flush=True)
+    assert hip.host_hip_peak() <= budget
+    w.close()
+w = wave(FP64, nrhs=2, k=4.0, n=6000)
+m = w.memory()
+w.close()
+# passes of one with packed operators, of two without
+w = wave(FP64, nrhs=2, k=4.0, n=6000, budget=m["fixed_bytes"] + 1.9 * m["per_rhs_bytes"])
+s = w.memory()
+assert s["slab"] == 2 and s["fixed_bytes"] < m["fixed_bytes"], (m, s)
+w.close()
+hip.host_hip_free_bytes(m["fixed_bytes"] + 2 * m["per_rhs_bytes"])      # not the window too
+hip.host_hip_reset()
+w = wave(FP64, nrhs=2, k=4.0, n=6000)
+s = w.memory()
+assert s["slab"] == 2 and s["fixed_bytes"] < m["fixed_bytes"], (m, s)
+assert hip.host_hip_peak() <= m["fixed_bytes"] + 2 * m["per_rhs_bytes"]
+w.close()
 """)
