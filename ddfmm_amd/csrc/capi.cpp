@@ -100,6 +100,13 @@ struct ddfmm_ctx {
         if (p) HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
         return p;
     }
+    // The last evaluation's end, also where it runs on a caller's stream: its graph and
+    // buffers are not touched before.
+    void wait() {
+        if (stream) (void)hipStreamSynchronize(stream);
+        if (aux) (void)hipStreamSynchronize(aux);
+        if (done_recorded) (void)hipEventSynchronize(done_ev);
+    }
     void drop_graphs() {
         for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
         graphs.clear();
@@ -172,8 +179,7 @@ int ddfmm_destroy(ddfmm_ctx* c) {
     if (!c) return DDFMM_OK;
     if (c->device >= 0) {
         (void)hipSetDevice(c->device);
-        if (c->stream) (void)hipStreamSynchronize(c->stream);
-        if (c->aux) (void)hipStreamSynchronize(c->aux);
+        c->wait();
         c->release();
         for (auto e : c->sync_ev)
             if (e) (void)hipEventDestroy(e);
@@ -250,6 +256,7 @@ static int setup_common(ddfmm_ctx* c, const double* pos, int64_t n, const ddfmm_
         if (c->device >= 0) {
             HIPCHK(hipSetDevice(c->device));
             HIPCHK(hipStreamSynchronize(c->stream));
+            c->wait();
         }
         c->release();
         c->hp = HostPlan();
@@ -527,7 +534,7 @@ int ddfmm_set_graph(ddfmm_ctx* c, int on) {
     if (!c) return fail(DDFMM_EINVAL, "null argument");
     if (!on && c->device >= 0) {
         (void)hipSetDevice(c->device);
-        if (c->stream) (void)hipStreamSynchronize(c->stream);
+        c->wait();
         c->drop_graphs();
     }
     c->use_graph = on != 0;
@@ -535,11 +542,11 @@ int ddfmm_set_graph(ddfmm_ctx* c, int on) {
 }
 
 // ---------------------------------------------------------------- GEMM tile autotuning
-// Upload the host tiles after a rebuild: the device table is replaced (the context's
-// stream is idle), the captured graphs are dropped and the stage times reset.
+// Upload the host tiles after a rebuild: the device table is replaced (no evaluation is in
+// flight), the captured graphs are dropped and the stage times reset.
 static void upload_tiles(ddfmm_ctx* c) {
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipStreamSynchronize(c->aux));
+    c->wait();
     auto it = std::find(c->allocs.begin(), c->allocs.end(), (void*)c->dp.tiles);
     if (it != c->allocs.end()) {
         HIPCHK(hipFree(*it));

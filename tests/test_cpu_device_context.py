@@ -138,3 +138,32 @@ assert s["slab"] == 2 and s["fixed_bytes"] < m["fixed_bytes"], (m, s)
 assert hip.host_hip_peak() <= m["fixed_bytes"] + 2 * m["per_rhs_bytes"]
 w.close()
 """)
+
+
+@pytest.mark.parametrize("end", ["w.close()", "w.set_graph(False)", "w.set_tiles([3] * len(w.tiles()[0]))",
+                                 "setup_again(w)", "w.autotune(1, 1)"])
+def test_graphs_live_until_their_replays_end(run, end):
+    """A replay on the caller's stream is waited for before its graph is destroyed, whatever
+    drops it."""
+    run(f"""
+from ddfmm_amd._lib import Hip, Params, check
+hip.hipStreamCreateWithFlags.argtypes = [ctypes.c_void_p, ctypes.c_uint]
+st = ctypes.c_void_p()
+hip.hipStreamCreateWithFlags(ctypes.byref(st), 1)
+
+def setup_again(w):
+    pos = np.ascontiguousarray(w.posptr)
+    prm = Params(K=K, ACCU=2, NPQ=4, ptsmax=100, maxlevel=12, numC=1, kernel=0, nrhs_max=1, precision=MIXED)
+    check(lib().ddfmm_setup_mlib(w._ctx, pos.ctypes.data, N, ctypes.byref(prm), ml.handle))
+
+w = wave(MIXED)
+w.set_graph(True)
+den, val = np.zeros(N, complex), np.zeros(N, complex)
+hip.host_hip_reset()
+w.eval_device(den.ctypes.data, val.ctypes.data, 1, st.value)
+{end}
+print("graphs destroyed in flight:", hip.host_hip_early(), flush=True)
+assert hip.host_hip_early() == 0
+w.close()
+assert hip.host_hip_live() == 0
+""")
