@@ -10,6 +10,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/ddfmm.h"
@@ -67,6 +68,7 @@ struct ddfmm_ctx {
     hipEvent_t sync_ev[STAGE_EVENTS] = {};     // fork/join events between the two streams
     hipEvent_t done_ev = nullptr;              // end of the last evaluation (on its stream)
     bool done_recorded = false;
+    int last_nrhs = 1;                         // right-hand sides of the last pass
     bool use_graph = false;                    // replay a captured graph of the stage sequence
     std::map<int, hipGraphExec_t> graphs;      // one per right-hand-side count
     size_t tiles_bytes = 0;                    // device bytes of the GEMM tile table
@@ -466,6 +468,7 @@ static int run_eval(ddfmm_ctx* c, const double2* den, double2* val, int nrhs, hi
     const auto& stages = c->hp.stages;
     if (c->done_recorded) HIPCHK(hipStreamWaitEvent(st, c->done_ev, 0));
     HIPCHK(launch_set_io(c->dp.io, den, val, st));
+    c->last_nrhs = nrhs;
     if (c->use_graph && !c->timing) {
         hipGraphExec_t x = graph_for(c, nrhs);
         HIPCHK(hipGraphLaunch(x, st));
@@ -770,19 +773,23 @@ int ddfmm_read_buffer(ddfmm_ctx* c, int buf, int rhs, int64_t off, int64_t count
     if (buf < 0 || buf >= BUF_COUNT || rhs < 0 || rhs >= c->slab || off < 0 || count < 0 ||
         off + count > c->hp.bufsize[buf])
         return fail(DDFMM_EINVAL, "buffer range out of bounds");
+    // the spectra of a pass hold its right-hand sides side by side, other buffers in slabs
+    const bool spectra = buf == BUF_SPEC || buf == BUF_TSPEC;
+    const int64_t step = spectra ? c->last_nrhs : 1;
+    if (spectra && rhs >= c->last_nrhs) return fail(DDFMM_EINVAL, "right-hand side not in the last pass");
     if (count == 0) return DDFMM_OK;
     try {
         HIPCHK(hipSetDevice(c->device));
         HIPCHK(hipStreamSynchronize(c->stream));
-        if (c->dp.mixed) {
-            std::vector<float2> tmp((size_t)count);
-            HIPCHK(hipMemcpy(tmp.data(), (float2*)c->dp.bt.p[buf] + (int64_t)rhs * c->hp.bufsize[buf] + off,
-                             (size_t)count * sizeof(float2), hipMemcpyDeviceToHost));
-            for (int64_t i = 0; i < count; ++i) { out[2 * i] = tmp[i].x; out[2 * i + 1] = tmp[i].y; }
-        } else {
-            HIPCHK(hipMemcpy(out, (double2*)c->dp.bt.p[buf] + (int64_t)rhs * c->hp.bufsize[buf] + off,
-                             (size_t)count * sizeof(double2), hipMemcpyDeviceToHost));
-        }
+        const int64_t first = spectra ? off * step + rhs : (int64_t)rhs * c->hp.bufsize[buf] + off;
+        const int64_t n = (count - 1) * step + 1;
+        auto read = [&](auto* from) {
+            std::vector<std::remove_const_t<std::remove_pointer_t<decltype(from)>>> tmp((size_t)n);
+            HIPCHK(hipMemcpy(tmp.data(), from + first, (size_t)n * sizeof(tmp[0]), hipMemcpyDeviceToHost));
+            for (int64_t i = 0; i < count; ++i) { out[2 * i] = tmp[i * step].x; out[2 * i + 1] = tmp[i * step].y; }
+        };
+        if (c->dp.mixed) read((const float2*)c->dp.bt.p[buf]);
+        else read((const double2*)c->dp.bt.p[buf]);
     } catch (const std::exception& e) {
         return fail(DDFMM_EDEVICE, e.what());
     }

@@ -167,7 +167,7 @@ DDFMM_API int ddfmm_get_stats(ddfmm_ctx* ctx, ddfmm_stats* st);
 DDFMM_API int ddfmm_dump_lists(ddfmm_ctx* ctx, char* buf, int64_t cap, int64_t* len);
 /* Inspection: copy `count` complex entries of internal vector buffer `buf` (leaf-sorted
    densities/potentials, LF/HF equivalent densities and check values; numbering of
-   ddfmm_amd/csrc/plan.hpp) for right-hand side `rhs`, starting at `off`. */
+   ddfmm_amd/csrc/plan.hpp) for right-hand side `rhs` of the last pass, starting at `off`. */
 DDFMM_API int ddfmm_read_buffer(ddfmm_ctx* ctx, int buf, int rhs, int64_t off, int64_t count, double* out);
 /* Per-stage timing: enable, then read, per stage of the last eval, its name, milliseconds
    (HIP events on the evaluation stream), algorithmic work per RHS (GEMM: useful complex
