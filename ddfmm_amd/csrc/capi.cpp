@@ -781,6 +781,7 @@ int ddfmm_read_buffer(ddfmm_ctx* c, int buf, int rhs, int64_t off, int64_t count
     try {
         HIPCHK(hipSetDevice(c->device));
         HIPCHK(hipStreamSynchronize(c->stream));
+        c->wait();
         const int64_t first = spectra ? off * step + rhs : (int64_t)rhs * c->hp.bufsize[buf] + off;
         const int64_t n = (count - 1) * step + 1;
         auto read = [&](auto* from) {

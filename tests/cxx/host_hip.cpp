@@ -5,6 +5,7 @@
 //   host_hip_fail(n)                the n-th fallible call from now fails (0: none)
 //   host_hip_calls                  fallible calls since host_hip_reset
 //   host_hip_early                  graphs destroyed before the host knew their last launch done
+//   host_hip_reads                  copies to the host while some stream was not known to be done
 //   host_hip_version(v)             the runtime version reported
 //   host_hip_free_bytes(n)          the free device memory reported
 // g++ -shared -fPIC -Wl,-soname,libamdhip64.so.7 -Wl,--version-script=host_hip.map
@@ -29,7 +30,7 @@ struct Exec {
 };
 std::map<void*, size_t> blocks;
 std::map<Stream*, int> streams;
-int64_t live = 0, peak = 0, calls = 0, fail_in = 0, early = 0, free_bytes = int64_t(1) << 40;
+int64_t live = 0, peak = 0, calls = 0, fail_in = 0, early = 0, reads = 0, free_bytes = int64_t(1) << 40;
 int last = 0, version = 70200000;
 Stream null_stream;
 
@@ -51,12 +52,13 @@ int64_t host_hip_live() { return live; }
 int64_t host_hip_peak() { return peak; }
 int64_t host_hip_calls() { return calls; }
 int64_t host_hip_early() { return early; }
+int64_t host_hip_reads() { return reads; }
 void host_hip_fail(int64_t n) { fail_in = n; }
 void host_hip_version(int v) { version = v; }
 void host_hip_free_bytes(int64_t n) { free_bytes = n; }
 void host_hip_reset() {
     peak = live;
-    calls = early = fail_in = 0;
+    calls = early = reads = fail_in = 0;
     last = 0;
 }
 
@@ -85,8 +87,10 @@ int hipFree(void* p) {
     std::free(p);
     return 0;
 }
-int hipMemcpy(void* d, const void* s, size_t n, int) {
+int hipMemcpy(void* d, const void* s, size_t n, int kind) {
     if (int e = err()) return e;
+    if (kind == 2)
+        for (auto& x : streams) reads += x.first->done < x.first->issued;
     std::memcpy(d, s, n);
     return 0;
 }

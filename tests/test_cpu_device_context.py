@@ -15,7 +15,7 @@ pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not ava
 PRELUDE = """
 import ctypes, sys
 hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-for f in ("live", "peak", "calls", "early"):
+for f in ("live", "peak", "calls", "early", "reads"):
     getattr(hip, "host_hip_" + f).restype = ctypes.c_int64
 for f in ("fail", "free_bytes"):
     getattr(hip, "host_hip_" + f).argtypes = [ctypes.c_int64]
@@ -166,4 +166,20 @@ print("graphs destroyed in flight:", hip.host_hip_early(), flush=True)
 assert hip.host_hip_early() == 0
 w.close()
 assert hip.host_hip_live() == 0
+""")
+
+
+def test_buffers_are_read_after_the_evaluation(run):
+    """ddfmm_read_buffer waits for an evaluation on a caller's stream."""
+    run("""
+hip.hipStreamCreateWithFlags.argtypes = [ctypes.c_void_p, ctypes.c_uint]
+st = ctypes.c_void_p()
+hip.hipStreamCreateWithFlags(ctypes.byref(st), 1)
+w = wave(MIXED)
+den, val = np.zeros(N, complex), np.zeros(N, complex)
+hip.host_hip_reset()
+w.eval_device(den.ctypes.data, val.ctypes.data, 1, st.value)
+w.read_buffer(2, 0, 10)
+assert hip.host_hip_reads() == 0, hip.host_hip_reads()
+w.close()
 """)
