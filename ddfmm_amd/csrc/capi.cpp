@@ -535,6 +535,16 @@ int ddfmm_eval_device(ddfmm_ctx* c, const void* den_dev, void* val_dev, int nrhs
 
 int ddfmm_set_graph(ddfmm_ctx* c, int on) {
     if (!c) return fail(DDFMM_EINVAL, "null argument");
+    if (on && c->device >= 0) {
+        // A process that runs on an older HIP runtime than this library is built for has
+        // crashed on the host during replays, the cause not known: none there.
+        int v = 0;
+        (void)hipRuntimeGetVersion(&v);
+        if (v / 100000 < HIP_VERSION / 100000)
+            return fail(DDFMM_ESTATE, "graph replay needs the HIP runtime " + std::to_string(HIP_VERSION_MAJOR) + "." +
+                                          std::to_string(HIP_VERSION_MINOR) + " that the library is built for, this process has loaded " +
+                                          std::to_string(v / 10000000) + "." + std::to_string(v / 100000 % 100));
+    }
     if (!on && c->device >= 0) {
         (void)hipSetDevice(c->device);
         c->wait();

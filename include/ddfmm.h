@@ -107,7 +107,8 @@ DDFMM_API int ddfmm_eval_device(ddfmm_ctx* ctx, const void* den_dev, void* val_d
    drops the graphs and issues the stages one by one again.  Timed evaluations
    (ddfmm_set_timing) always issue the stages one by one.  No counterpart in the
    reference (which has no device); results are bit-identical to the stage-by-stage
-   path. */
+   path.  Refused (DDFMM_ESTATE) where the process has loaded an older HIP runtime than
+   the library is built for. */
 DDFMM_API int ddfmm_set_graph(ddfmm_ctx* ctx, int on);
 
 /* GEMM tile autotuning (no counterpart in the reference).  Every planned GEMM stage

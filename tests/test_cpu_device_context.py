@@ -183,3 +183,28 @@ w.read_buffer(2, 0, 10)
 assert hip.host_hip_reads() == 0, hip.host_hip_reads()
 w.close()
 """)
+
+
+def test_graph_replay_needs_the_runtime_it_was_built_for(run):
+    """An older HIP runtime in the process (one bundled with another package and loaded first)
+    is refused when replay is switched on; the stage-by-stage path stays."""
+    run("""
+w = wave(MIXED)
+den, val = np.zeros(N, complex), np.zeros(N, complex)
+hip.host_hip_version(70051831)
+try:
+    w.set_graph(True)
+    assert False, "accepted"
+except DdfmmError as e:
+    assert "7.0" in str(e) and "runtime" in str(e), str(e)
+w.set_graph(False)
+w.eval(den)
+for v in (70200000, 70351831, 80000000):
+    hip.host_hip_version(v)
+    w.set_graph(True)
+w.eval(den)
+w.close()
+host = wave(MIXED, device=-1)
+hip.host_hip_version(70051831)
+host.set_graph(True)
+""")
