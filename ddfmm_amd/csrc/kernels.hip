@@ -999,6 +999,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     }
 }
 
+// Tallest tiles of a form: with two column blocks, seven row blocks take all 256 registers and
+// spill.
+constexpr int gemm_max_mb(int cb) { return cb > 1 ? GEMM_MB - 1 : GEMM_MB; }
+
 // From 16 right-hand sides up, where a wave's 16 columns are one box's and tiles fill whole
 // waves, each FP32 wave is a block of its own: the waves share nothing but cache lines, and a
 // block of four is not placed before a slot is free on every SIMD, nor its slots reused before
@@ -1012,8 +1016,10 @@ void launch_gemm_form(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d
     const dim3 grid((s.end - s.begin) * ((nrhs + CB - 1) / CB) * (one ? 4 : 1), 1), block(one ? 64 : 256);
 #define DDFMM_GEMM_MB(X)                                                                                            \
     case X:                                                                                                         \
-        gemm_kernel<TA, V, R, X, CB, PACK, G3M><<<grid, block, 0, st>>>(d.groups, d.tiles, d.colB, d.colC, d.colA,  \
-                                                                        opm, d.opmat, d.zeros, d.bt, s.begin, nrhs); \
+        if constexpr (X <= gemm_max_mb(CB))                                                                         \
+            gemm_kernel<TA, V, R, X, CB, PACK, G3M><<<grid, block, 0, st>>>(d.groups, d.tiles, d.colB, d.colC,      \
+                                                                            d.colA, opm, d.opmat, d.zeros, d.bt,    \
+                                                                            s.begin, nrhs);                         \
         break;
     switch (s.mb) {
         DDFMM_GEMM_MB(1) DDFMM_GEMM_MB(2) DDFMM_GEMM_MB(3) DDFMM_GEMM_MB(4) DDFMM_GEMM_MB(5)
@@ -1030,15 +1036,21 @@ void launch_gemm64(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
 
 // FP32 products on packed operators.  Two column blocks per wave (CB = 2) halve the operator
 // traffic per product but leave two waves per SIMD and take the union of twice the columns'
-// K blocks: they pay where K is not blocked and the columns of a box fill a wave (32 RHS and
-// up; M2L and W > 1 L2L at 64 RHS 13.7 -> 13.2 ms, at 8 and 16 RHS the same or slower, K-blocked
-// U2U 17.3 -> 18.1 ms) and the launch still has four blocks per CU.
+// K blocks.  They pay with three products per complex one, where K is not blocked and the
+// columns of a box fill a wave, and the launch still has four blocks per CU: all translations
+// of 250k points at 24, 32, 48 and 64 RHS, one block -> two, 17.3 -> 17.15, 22.75 -> 22.4, 34.6 -> 34.0
+// and 44.9 -> 44.0 ms; at 8 and 16 RHS the same or slower, K-blocked U2U at 64 RHS 17.3 -> 18.1.  With
+// four products the matrix cores are the longer part: 35.3 -> 35.6, 46.1 -> 46.6, 69.4 -> 69.8 and 91.2 ->
+// 91.7 ms, so those keep one.
 template <bool G3M>
 void launch_gemm32(const Stage& s, int nrhs, hipStream_t st, const DevPlan& d) {
-    if (nrhs >= 32 && !s.kblocked && (int64_t)(s.end - s.begin) * nrhs / 2 >= 1024 && s.mb < GEMM_MB)
-        launch_gemm_form<float2, float2, float, 2, true, G3M>(s, nrhs, st, d, d.oppack);
-    else
-        launch_gemm_form<float2, float2, float, 1, true, G3M>(s, nrhs, st, d, d.oppack);
+    if constexpr (G3M) {
+        if (nrhs >= 32 && !s.kblocked && (int64_t)(s.end - s.begin) * nrhs / 2 >= 1024 && s.mb <= gemm_max_mb(2)) {
+            launch_gemm_form<float2, float2, float, 2, true, G3M>(s, nrhs, st, d, d.oppack);
+            return;
+        }
+    }
+    launch_gemm_form<float2, float2, float, 1, true, G3M>(s, nrhs, st, d, d.oppack);
 }
 
 // Blocks per kernel matrix or packed operator block at setup: a setup window holds a few
