@@ -617,7 +617,7 @@ int ddfmm_autotune(ddfmm_ctx* c, int nrhs, int reps, int cap, int* mbmax, int* c
         HIPCHK(hipMemsetAsync(c->dp.host_io, 0, (size_t)c->hp.N * nrhs * sizeof(double2), c->stream));
         std::vector<int> cur(nl);
         for (int l = 0; l < nl; ++l) cur[l] = c->hp.lgemm[l].mbmax;
-        // the planner's tiling (height limit GEMM_MB, rows split further for small stages)
+        // the planner's own tiling
         std::vector<double> t0 = time_logical(c, nrhs, reps);
         std::vector<int> best = cur;
         std::vector<double> bt = t0;

@@ -671,7 +671,23 @@ template <> struct Mfma<double> {
 
 constexpr int MAXKB = 8;           // at most 8 K blocks (children of a box)
 
-// C[:, ccol] (=|+=) diag(scale) * op(A) * B[:, bcol] on MFMA 16x16x4 (f32 or f64).
+// Two adjacent FP32 complex values by one 16-byte load (global loads need dword alignment
+// only).
+struct CPair {
+    float2 e[2];
+};
+__device__ __forceinline__ CPair load_pair(const float2* p) {
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
+    const f4u r = *(const f4u*)p;
+    return {{make_float2(r.x, r.y), make_float2(r.z, r.w)}};
+}
+
+// Units (8 k in FP32, 4 in FP64) per pipeline step: short tiles run few MFMAs per unit, so
+// they load further ahead.  U2U of 6k points in FP64 (858 waves of one row block) 0.123 -> 0.104
+// ms, of 60k 0.39 -> 0.35; twice as many units at one and two row blocks: 0.103 and 0.37.
+constexpr int gemm_units(int mb, int cb) { return cb > 1 || mb > 3 ? 1 : mb > 1 ? 2 : 4; }
+
+// C[:, ccol] (=|+=) diag(scale) * A * B[:, bcol] on MFMA 16x16x4 (f32 or f64).
 // A block covers MB row blocks of 16 (the group's rows split evenly over its tiles; tiles
 // are launched per MB) and 64 CB columns; each of its four waves owns 16 CB columns and
 // works alone: operands go straight from memory (A from L2 and L1, where the block's waves
@@ -701,22 +717,7 @@ constexpr int MAXKB = 8;           // at most 8 K blocks (children of a box)
 // multiplies is the block's own); row blocks past the group's last one are never read, rows
 // past it not stored.  A column's order of k depends on G3M alone, so neither MB nor CB changes a
 // bit (the instruction itself sums its k in order by fma).
-// Two adjacent FP32 complex values by one 16-byte load (global loads need dword alignment
-// only).
-struct CPair {
-    float2 e[2];
-};
-__device__ __forceinline__ CPair load_pair(const float2* p) {
-    typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
-    const f4u r = *(const f4u*)p;
-    return {{make_float2(r.x, r.y), make_float2(r.z, r.w)}};
-}
-
-// Units (8 k in FP32, 4 in FP64) per pipeline step: short tiles run few MFMAs per unit, so
-// they load further ahead.  U2U of 6k points in FP64 (858 waves of one row block) 0.123 -> 0.104
-// ms, of 60k 0.39 -> 0.35; twice as many units at one and two row blocks: 0.103 and 0.37.
-constexpr int gemm_units(int mb, int cb) { return cb > 1 || mb > 3 ? 1 : mb > 1 ? 2 : 4; }
-
+//
 // PACK: A packed (PackA in plan.hpp) in the order the lanes take it; else as stored in the
 // operator table (the setup's products, FP64 contexts whose budget holds no packed copy).
 template <class TA, class V, class R, int MB, int CB, bool PACK, bool G3M>
@@ -1949,11 +1950,6 @@ __global__ __launch_bounds__(256) void reduce_kernel(const RTarget* __restrict__
     }
 }
 
-// Grid caps of the launches on the second stream (multiples of 8: one XCD round), for
-// running them as a background beside the GEMMs; very large = one block per item
-constexpr int AUX_KAPPLY_BLOCKS = 1 << 30;
-constexpr int AUX_BLOCKS = 1 << 30;
-
 int grid_for(int64_t n, int threads) {
     int64_t b = (n + threads - 1) / threads;
     return (int)std::min<int64_t>(std::max<int64_t>(b, 1), 65536);
@@ -1976,10 +1972,9 @@ hipError_t launch_stage_t(const DevPlan& d, const Stage& s, int nrhs, hipStream_
                                                                      nrhs);
         break;
     case ST_KAPPLY: {
-        const int gx = s.stream ? std::min(n, AUX_KAPPLY_BLOCKS) : n;
         if constexpr (sizeof(V) == 8) if (d.kmfma) {   // mixed precision: the products on the matrix cores
             const int nb = nrhs > 8 ? 2 : 1;
-            const dim3 grid(gx, (nrhs + 8 * nb - 1) / (8 * nb));
+            const dim3 grid(n, (nrhs + 8 * nb - 1) / (8 * nb));
 #define DDFMM_KMFMA(NB, KT, MIR) \
     kapply_mfma_kernel<NB, KT, MIR><<<grid, 256, 0, st>>>(d.ktasks, d.ksrcs, d.px, d.py, d.pz, d.bt, s.begin, n, nrhs)
             const int sel = (nb == 2 ? 4 : 0) + (d.ktype ? 2 : 0) + (s.mb == 1 ? 1 : 0);
@@ -1998,8 +1993,8 @@ hipError_t launch_stage_t(const DevPlan& d, const Stage& s, int nrhs, hipStream_
         }
         if (s.mb == 1) return hipErrorInvalidValue;    // mirror slots need the matrix-core kernel
 #define DDFMM_KAPPLY(RC, KT) \
-    kapply_kernel<V, RC, KT><<<dim3(gx, (nrhs + RC - 1) / RC), KA_THREADS, 0, st>>>(d.ktasks, d.ksrcs, d.px, d.py, \
-                                                                                    d.pz, d.bt, s.begin, n, nrhs)
+    kapply_kernel<V, RC, KT><<<dim3(n, (nrhs + RC - 1) / RC), KA_THREADS, 0, st>>>(d.ktasks, d.ksrcs, d.px, d.py, \
+                                                                                   d.pz, d.bt, s.begin, n, nrhs)
         // G(t, s) evaluated once for up to 1, 4 or 8 right-hand sides
         switch ((nrhs == 1 ? 0 : nrhs <= 4 ? 2 : 4) + (d.ktype ? 1 : 0)) {
         case 0: DDFMM_KAPPLY(1, 0); break;
@@ -2028,10 +2023,11 @@ hipError_t launch_stage_t(const DevPlan& d, const Stage& s, int nrhs, hipStream_
     case ST_FFTFWD:
         if (d.P != 6) return hipErrorInvalidValue;
         if (nrhs == 1) {
-            fft_fwd_kernel<V><<<dim3(s.stream ? std::min(n, AUX_BLOCKS) : n, 1), 256, 0, st>>>(d.fsrc, d.grid, d.NL,
-                                                                                           d.bt, s.begin, n, 1);
-        } else {    // 8 (FP32) or 4 (FP64) right-hand sides per block, two at a time: 66 or 76 KB
-            // of LDS (an FP32 block still fits beside two translation-GEMM blocks)
+            fft_fwd_kernel<V><<<dim3(n, 1), 256, 0, st>>>(d.fsrc, d.grid, d.NL, d.bt, s.begin, n, 1);
+        } else {    // 8 (FP32) or 4 (FP64) right-hand sides per block, two at a time: 66 or 76 KB of
+            // LDS.  One and four at a time: 250k x 64 alone 2.64 and 1.98 ms (two 2.39), the pass
+            // 66.4 and 66.0 (66.05); 1M x 2 0.29 and 0.244 (0.239).  Beside the GEMMs the FFT is
+            // hidden, so the block that takes less LDS stays.
             constexpr int R = sizeof(V) == 8 ? 8 : 4;
             fft_fwd_multi_kernel<V, R, 2><<<dim3(n, (nrhs + R - 1) / R), 256, 0, st>>>(d.fsrc, d.grid, d.NL, d.bt,
                                                                                  s.begin, n, nrhs);

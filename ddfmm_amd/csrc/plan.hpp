@@ -71,7 +71,7 @@ struct KTask {
 // matching A column block at colA[acol0 + block] (used to concatenate the non-empty
 // children of a box along K without padding).
 struct GGroup {
-    int64_t aoff;   // A offset in the operator table
+    int64_t aoff;   // A offset in the operator table, or in the packed one
     int64_t soff;   // row scale (length M) offset, or -1
     int M, K, lda, transA;      // transA: 0 A[m + k lda], 1 A[k + m lda], 2 / 3 packed FP32 / FP64
     int bbuf, cbuf;

@@ -25,8 +25,7 @@ struct PlanStats {
 };
 
 // A planned GEMM stage before it is cut into one launch per tile height: its groups, in
-// order, and the largest tile height its tiling uses (GEMM_MB, or less where rows were
-// split for a small stage).
+// order, and the largest tile height its tiling uses.
 struct LogicalGemm {
     std::vector<int> groups;
     int mbmax = GEMM_MB;

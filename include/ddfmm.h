@@ -115,7 +115,7 @@ DDFMM_API int ddfmm_set_graph(ddfmm_ctx* ctx, int on);
    (a translation level: U2U, M2L, D2D, LF M2M/L2L, solves) is tiled with at most
    mbmax row blocks of 16 per tile (1..7; a group's rows spread evenly over its tiles).
    ddfmm_autotune times, for nrhs right-hand sides, every stage under each limit 1..7
-   and under the planner's own tiling (limit 7, rows split further for small stages),
+   and under the planner's own tiling (a limit estimated per stage),
    one stage at a time on one stream (best of reps evaluations after a warm-up), keeps
    the fastest per stage and returns the per-stage limits in mbmax (count entries, up to
    cap) and the summed GEMM milliseconds before and after.  ddfmm_set_tiles applies a
