@@ -71,7 +71,7 @@ class GpuEngine:
 
     def __init__(self, key, pos, wave_opts, ops, nrhs_slot, precision, kernel=0, numC=1, hip=None,
                  autotune=True, graph=True):
-        from ._lib import Hip
+        from ._lib import DdfmmError, Hip
         from .wave3d import Kernel3d, Mlib3d, Wave3d
 
         self.key = key
@@ -96,7 +96,10 @@ class GpuEngine:
             else:
                 self.w.set_tiles(self.tiles)
         if graph:
-            self.w.set_graph(True)
+            try:
+                self.w.set_graph(True)
+            except DdfmmError:      # the process runs on an older HIP runtime than replay needs:
+                pass                # stage by stage, the same bits
         self.stream = self.hip.stream()
         nb = nrhs_slot * self.N * 16
         self.slots = []

@@ -208,3 +208,23 @@ host = wave(MIXED, device=-1)
 hip.host_hip_version(70051831)
 host.set_graph(True)
 """)
+
+
+def test_serving_engine_runs_without_replay_on_an_older_runtime(run):
+    """An engine asks for graph replay by default; where the process's HIP runtime is too old
+    for it, the engine evaluates stage by stage."""
+    run("""
+from ddfmm_amd.serve import GpuEngine
+
+class Buffers:
+    stream = event = lambda self: 0
+    pinned = malloc = lambda self, n: n
+
+opts = {"-wave3d_ACCU": 2, "-wave3d_K": K, "-wave3d_maxlevel": 12}
+for v in (70051831, 70200000):
+    hip.host_hip_version(v)
+    e = GpuEngine("g", geometry.sphere(N, K, 81), opts, (sys.argv[3], sys.argv[4]), 2, MIXED, hip=Buffers(),
+                  autotune=False)
+    e.w.eval(np.zeros(N, complex))
+    e.w.close()
+""")
