@@ -127,8 +127,6 @@ KNAME = {
     else "gemm_kernel<double2,double2,double>",
     "gemm_solve": lambda vt, n: "gemm_kernel<double2,float2,double>" if vt == "float2"
     else "gemm_kernel<double2,double2,double>",
-    "kapply": lambda vt, n: f"kapply_kernel<{vt},{rhs_block(n)}>",
-    "kapply_mfma": lambda nb, kt: f"kapply_mfma_kernel<{nb},{kt},false>",
     "vlist": _vlist_name,
     "fft_fwd": lambda vt, n: f"fft_fwd_kernel<{vt}>" if n == 1 else
     f"fft_fwd_multi_kernel<{vt},{8 if vt == 'float2' else 4},2>",
@@ -256,8 +254,9 @@ def stage_detail(w, st, dd, vd, nrhs, precision, workload, kernel=0):
     vt = "float2" if mixed else "double2"
     kname = KNAME.get(dom, lambda vt, n: dom)(vt, nrhs)
     kmfma = mixed and nrhs >= 4         # contexts of >= 4 RHS apply kernels on the matrix cores
-    if dom == "kapply" and kmfma:
-        kname = KNAME["kapply_mfma"](2 if nrhs > 8 else 1, kernel)
+    if dom == "kapply":
+        kname = (f"kapply_mfma_kernel<{2 if nrhs > 8 else 1},{kernel},false>" if kmfma else
+                 f"kapply_kernel<{vt},{rhs_block(nrhs)},{kernel}>")
     if dom in ("gemm_translation", "gemm_solve"):
         peak = PEAK["fp32"] if (mixed and dom == "gemm_translation") else PEAK["fp64"]
         work_desc = "useful complex-GEMM flops 8*M*K*N over the class's groups"
