@@ -695,20 +695,22 @@ constexpr int gemm_units(int mb, int cb) { return cb > 1 || mb > 3 ? 1 : mb > 1 
 // and no barriers.  K runs over segments: the whole K, or the K blocks present in at least
 // one of the wave's columns.
 //
-// What bounds it: the vector memory path.  With its loads taken out the loop runs at 143 of
-// the 155 TF/s that the f32 matrix cores sustain here; A in the stored order (ten 8-byte
-// loads per 30 MFMAs, each over four half-filled line groups) held it at 98, packed A (five
-// 16-byte loads of a contiguous KiB) brings it to 120.  Staging through LDS (two buffers,
-// one barrier per 16 k) reached 85 to 101: 124 with neither loads nor stores, as its waves
-// stall together at the barriers.  Translations alone, LDS form -> this one: 4M points x 8
-// RHS 28.9 -> 23.4 ms, 250k x 64 RHS 58.9 -> 43.7 ms, 1M x 1 RHS 5.9 -> 4.5 ms.
+// What bounds it: loads first, then the ends of segments and launches.  4M points x 8 RHS on
+// one stream: the translations take 23.2 ms, the matrix cores busy 65% of it (101 TF/s, padding
+// included, of the 155 that they sustain); with the operands of a wave's first step in place
+// of all later loads 18.8 ms (125 TF/s).  250k x 64 RHS 42.9 and 34.7 ms, 1M x 1 RHS 4.41 and 3.57.
+// A in the stored order (ten 8-byte loads per 30 MFMAs, each over four half-filled line groups,
+// where packed A takes five 16-byte loads of a contiguous KiB) reached 0.82 of this rate.
+// Staged through LDS (two buffers, one barrier per 16 k), the waves stall together at the
+// barriers; LDS form -> this one: 4M x 8 28.9 -> 23.4 ms, 250k x 64 58.9 -> 43.7, 1M x 1 5.9 -> 4.5.
 //
-// Launches of a wave or less per SIMD are bound by that wave's own instructions: beside 106
-// ns of FP64 (40 of FP32) MFMAs a k step of one row block took 80 (65) ns of address
-// arithmetic, clamps and selects, which only other waves can hide.  So little of that is left
-// in a step: absent blocks and columns point to a block of zeros, and the loads run up to a
-// step past a segment's end, at constant offsets from one pointer per column block.  FP64 U2U
-// of 6k points 0.105 -> 0.084 ms, of 60k 0.35 -> 0.30, 1M x 1 RHS 2.04 -> 1.95.
+// Launches of a wave or less per SIMD are bound by that wave's own instructions: beside the
+// MFMAs of a k step of one row block (106 ns in FP64, 40 in FP32) stands its address
+// arithmetic, which only other waves can hide.  So little of that is left in a step: absent
+// blocks and columns point to a block of zeros, and the loads run up to a step past a segment's
+// end, at constant offsets from one pointer per column block.  With clamps and selects in place
+// of that -> now: FP64 U2U of 6k points 0.105 -> 0.084 ms, of 60k 0.35 -> 0.30, 1M x 1 RHS 2.04 ->
+// 1.95.
 //
 // Bounds of the loads: B up to GEMM_AHEAD k past the segment, in the slack behind each
 // buffer at its end (BUF_SLACK; the zeros behind the operator table, the setup window's

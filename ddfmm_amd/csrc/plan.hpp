@@ -196,7 +196,7 @@ struct Stage {
                         // ST_KAPPLY: 1 when sources carry mirror slots (KSrc::moff)
     int lstage;         // ST_GEMM: logical stage (all tile heights of one planned GEMM stage), else -1
     int kblocked;       // ST_GEMM: the groups' K is blocked (GGroup::kb > 0)
-    double exec;        // ST_GEMM: MFMA flops per RHS the kernel executes (padding included)
+    double exec;        // ST_GEMM: MFMA flops of one RHS alone (padding included, four products)
     char name[24];
 };
 

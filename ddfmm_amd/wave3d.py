@@ -259,7 +259,8 @@ class Wave3d:
                  kinds[i] // 16) for i in range(n)]
 
     def stage_exec(self):
-        """Per stage, the MFMA flops per RHS the GEMM kernel executes (0 for other stages)."""
+        """Per stage, the MFMA flops an evaluation of one RHS executes in the GEMM kernel, four real
+        products per complex one (0 for other stages)."""
         cnt = ctypes.c_int()
         check(lib().ddfmm_stage_exec(self._ctx, 0, None, ctypes.byref(cnt)))
         ex = (ctypes.c_double * cnt.value)()

@@ -179,9 +179,11 @@ DDFMM_API int ddfmm_read_buffer(ddfmm_ctx* ctx, int buf, int rhs, int64_t off, i
 DDFMM_API int ddfmm_set_timing(ddfmm_ctx* ctx, int on);
 DDFMM_API int ddfmm_stage_times(ddfmm_ctx* ctx, int cap, char* names /* cap x 24 */, double* ms, double* work,
                       int* kinds, int* count);
-/* Per stage, the MFMA flops per RHS the GEMM kernel executes under its tiling (16-row
-   blocks, 16-column waves, 4-deep k steps, present K blocks only; 0 for other stages):
-   executed / useful work is the padding overhead.  No counterpart in the reference. */
+/* Per stage, the MFMA flops an evaluation of one RHS executes in the GEMM kernel under its
+   tiling (16-row blocks, 16-column waves, 4-deep k steps, present K blocks only, four real
+   products per complex one; 0 for other stages): executed / useful work is the padding
+   overhead.  More RHS execute less than that times their number, since a wave then covers
+   fewer boxes.  No counterpart in the reference. */
 DDFMM_API int ddfmm_stage_exec(ddfmm_ctx* ctx, int cap, double* exec, int* count);
 
 #ifdef __cplusplus
